@@ -39,10 +39,10 @@ _c_u8p = ctypes.POINTER(ctypes.c_uint8)
 
 
 def build(with_reference: bool | None = None) -> None:
-    """Compile liboracle.so and, when the reference tree is present, oracle/_ref."""
+    """Compile liboracle.so and, where the reference's sources are, oracle/_ref."""
     subprocess.run(["make", "-s", "-C", str(ORACLE_DIR)], check=True)
     if with_reference is None:
-        with_reference = REFERENCE_TREE.is_dir()
+        with_reference = (REFERENCE_TREE / "asdsl" / "kernels" / "native").is_dir()  # not an empty mount point
     if with_reference:
         subprocess.run(["make", "-s", "-C", str(ORACLE_DIR), "ref"], check=True)
 
