@@ -99,6 +99,8 @@ SIGNATURES: dict[str, list] = {
     "asdsl_decode_token_upto": [_P, _P, _P, _I, _P, _P, _P],
     "asdsl_decode_verify_work_bytes": [_P, _I],
     "asdsl_decode_verify": [_P, _P, _I, _P, _P, _P, _P, _P],
+    "asdsl_decode_prefill_work_bytes": [_P, _I],
+    "asdsl_decode_prefill": [_P, _P, _I, _I, _P, _P, _P, _P, _P],
     "asdsl_kv_zero_from": [_P, _P, _I, _I, _I, _I, _P],
     "asdsl_kv_zero_from_q8": [_P, _P, _P, _P, _I, _I, _I, _I, _P],
     "asdsl_repack_preq_to_preq2": [_P, _P, _P, _I, _I, _I, _P],
@@ -110,6 +112,7 @@ SIGNATURES: dict[str, list] = {
 }
 _RESTYPE = {"asdsl_last_error": ctypes.c_char_p, "asdsl_attention_work_floats": ctypes.c_size_t,
             "asdsl_decode_work_bytes": ctypes.c_size_t, "asdsl_decode_verify_work_bytes": ctypes.c_size_t,
+            "asdsl_decode_prefill_work_bytes": ctypes.c_size_t,
             "asdsl_decode_flags_offset": ctypes.c_size_t,
             "asdsl_sparse_down_work_bytes": ctypes.c_size_t, "asdsl_grid_sync_probe_work_bytes": ctypes.c_size_t,
             "asdsl_gemv_preq2_fused_batch_work_bytes": ctypes.c_size_t,

@@ -312,6 +312,8 @@ class DecodeEngine:
         self.kv_seq_len = 0
         self._kv_snapshots: list[int] = []
         self._verify = None  # work, token, logits and next-token buffers of the verify pass
+        self._prefill_work = None  # work buffer of a prefill chunk of up to _prefill_tokens tokens
+        self._prefill_tokens = 0
         # ASDSL_ENGINE_PROFILE / ASDSL_ENGINE_PROFILE_TOKEN, read like the
         # reference's engine_profile_enabled/_target_token
         # (asdsl/kernels/native/unified_engine.cpp:71-87): the target decode
@@ -475,14 +477,23 @@ class DecodeEngine:
     # it on the step's deep attention form splits differently.
     EXACT_BATCH_LIMIT = 2048
 
+    # tokens of one prefill chunk
+    MAX_PREFILL_TOKENS = 512
+
     def prefill(self, tokens) -> None:
         """The prompt tokens at positions 0, 1, ...: the K/V rows, the device
         token (the greedy token after the last one), the logits of the last
         token and the position that forward_token on each in turn leaves,
-        bit for bit; below EXACT_BATCH_LIMIT positions as verify passes of up
-        to MAX_VERIFY_TOKENS tokens (one pass instead of one step per token),
-        the rest as single steps."""
+        bit for bit.  From four tokens in chunks of up to MAX_PREFILL_TOKENS
+        (asdsl_decode_prefill).  Fewer tokens, and every prompt while one of
+        the switches is set that give the verify pass or the step another
+        arithmetic, run as verify passes of up to MAX_VERIFY_TOKENS tokens
+        below EXACT_BATCH_LIMIT positions and single steps beyond."""
         toks = [int(t) for t in tokens]
+        if len(toks) >= 4 and not any(os.environ.get(k, "") not in ("", "0") for k in (
+                "ASDSL_HIP_NORM_FACTORED", "ASDSL_HIP_VERIFY_MFMA", "ASDSL_HIP_VERIFY_DOT4")):
+            self._prefill_chunks(toks)
+            return
         pos = 0
         while pos < len(toks):
             n = min(self.MAX_VERIFY_TOKENS, len(toks) - pos, self.EXACT_BATCH_LIMIT - pos)
@@ -494,6 +505,36 @@ class DecodeEngine:
             else:
                 self.forward_token(toks[pos], pos)
                 pos += 1
+
+    def _prefill_chunks(self, toks: list[int]) -> None:
+        import torch
+
+        c = self.cfg
+        if any(not 0 <= t < c.vocab for t in toks):
+            raise ValueError("prefill: token_id out of vocab range")
+        if len(toks) > c.max_seq:
+            raise ValueError("prefill: positions out of kv-cache range")
+        most = min(len(toks), self.MAX_PREFILL_TOKENS)
+        if self._prefill_work is None or self._prefill_tokens < most:
+            # grown in steps, so that prompts of rising length allocate a few times only
+            most = min(max(most, 2 * self._prefill_tokens, 64), self.MAX_PREFILL_TOKENS)
+            nbytes = _hip.LIB.asdsl_decode_prefill_work_bytes(ctypes.byref(self._model), most)
+            if nbytes == 0:
+                raise ValueError(f"invalid decode model: {_hip.last_error()}")
+            self._prefill_work = torch.empty(nbytes, dtype=torch.uint8, device=self.token.device)
+            self._prefill_tokens = most
+        ids = torch.tensor(toks, dtype=torch.int32).to(self.token.device)
+        stream = _hip.stream_handle()
+        for pos in range(0, len(toks), self.MAX_PREFILL_TOKENS):
+            n = min(self.MAX_PREFILL_TOKENS, len(toks) - pos)
+            last = pos + n == len(toks)
+            _hip.check(_hip.LIB.asdsl_decode_prefill(ctypes.byref(self._model), _hip.ptr(ids[pos:]), n, pos,
+                                                     _hip.ptr(self.token), _hip.ptr(self.pos),
+                                                     _hip.ptr(self.logits) if last else None,
+                                                     _hip.ptr(self._prefill_work), stream),
+                       "asdsl_decode_prefill")
+        self._host_pos = len(toks)
+        self.kv_seq_len = max(self.kv_seq_len, len(toks))
 
     def decode_steps(self, k: int) -> list[int]:
         """k greedy steps (step(), captured graphs) queued back to back from

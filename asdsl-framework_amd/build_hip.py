@@ -47,6 +47,7 @@ COMMON_FLAGS = [
 # 16-column prefetching instance: 3228 -> 2841 instructions).
 FILE_FLAGS = {
     "gemv_preq2_batch.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
+    "gemm_preq2_exact.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
 }
 
 

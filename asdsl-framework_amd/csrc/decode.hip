@@ -22,6 +22,8 @@
 // launch.
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
 #include "abi_util.hpp"
 #include "device_common.hpp"
 
@@ -312,8 +314,8 @@ inline int combine_threads(int max_ns) {
 
 // IMG_GS (32 or 128): the head's 128 outputs of column c are also quantized
 // into the o_proj batched GEMV's int8 image (image_store8, 16 chunks per
-// head), and columns c >= ncols (the grid covers kImageCols columns) write
-// that image's zero columns.
+// head; column c's image is c / kImageCols), and columns c >= ncols write
+// that image's zero columns.  out may be null then.
 template <int IMG_GS>
 __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const float* __restrict__ part,
                                                                       const int* __restrict__ pos_ptr,
@@ -335,8 +337,15 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const flo
     const int g = tid / kHeadDim;
     // the first kHeadChunks lanes quantize the head's outputs (8 each)
     auto image_chunk = [&](const float (&v)[8]) {
-        if constexpr (IMG_GS != 0) image_store8<IMG_GS>(v, h * kHeadChunks + tid, col, true, img, fac, us);
+        if constexpr (IMG_GS != 0)
+            image_store8<IMG_GS>(v, h * kHeadChunks + tid, col % kImageCols, true, img, fac, us);
     };
+    if constexpr (IMG_GS != 0) {
+        const size_t at = image_at(col, static_cast<int>(gridDim.x) * kHeadDim);
+        img += at / sizeof(uint2);
+        fac += at / sizeof(float2);
+        us += at / sizeof(float);
+    }
     const float zeros[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (IMG_GS != 0 && col >= ncols) {
         if (tid < kHeadChunks) image_chunk(zeros);
@@ -344,9 +353,9 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const flo
     }
     const int pos = *pos_ptr + col;
     part += static_cast<size_t>(col) * gridDim.x * nsplit * kPartStride;
-    out += static_cast<size_t>(col) * gridDim.x * kHeadDim;
+    if (out) out += static_cast<size_t>(col) * gridDim.x * kHeadDim;
     if (pos < 0 || pos >= max_seq || pos >= pos_limit) {  // no partials were written (see attn_decode_kernel)
-        if (g == 0) out[static_cast<size_t>(h) * kHeadDim + d] = 0.0f;
+        if (g == 0 && out) out[static_cast<size_t>(h) * kHeadDim + d] = 0.0f;
         if (IMG_GS != 0 && tid < kHeadChunks) image_chunk(zeros);
         return;
     }
@@ -416,7 +425,7 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const flo
             res = sum * (1.0f / Ls);
         }
     }
-    if (g == 0) out[static_cast<size_t>(h) * kHeadDim + d] = res;
+    if (g == 0 && out) out[static_cast<size_t>(h) * kHeadDim + d] = res;
     if constexpr (IMG_GS != 0) {
         if (g == 0) res_s[d] = res;
         __syncthreads();
@@ -844,7 +853,7 @@ __global__ __launch_bounds__(256) void verify_embed_kernel(const uint16_t* __res
     for (int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); i < hidden;
          i += static_cast<int>(gridDim.x * blockDim.x))
         H[static_cast<size_t>(c) * hidden + i] = h2f(row[i]);
-    if (blockIdx.x == 0 && threadIdx.x == 0) keys[c] = 0ull;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && keys) keys[c] = 0ull;
 }
 
 // Per column c (one workgroup): h = H[c] + D[c] (D may be null), written back
@@ -856,8 +865,9 @@ __global__ __launch_bounds__(256) void verify_embed_kernel(const uint16_t* __res
 // 8 wave sums in order, so both passes normalize identically.
 // IMG_GS (32 or 128): X[c] is also quantized into the next batched GEMV's
 // int8 image (image_store8, the values batch_quantize_kernel would form from
-// X), and workgroups c >= ncols (the grid covers kImageCols columns) write
+// X; column c's image is c / kImageCols), and workgroups c >= ncols write
 // that image's zero columns, so the GEMV needs no quantize launch of its own.
+// X may be null then.
 // inv_out (IMG_GS = 0 only): the single-token GEMV's factored form instead,
 // X[c] = h * w and inv_out[c] = inv_rms, which the batched GEMV applies to
 // its reduced rows (preq2_batch_exact), as the norm-fed GEMV's prologue and
@@ -876,17 +886,21 @@ __global__ __launch_bounds__(kNormThreads) void verify_add_norm_kernel(float* __
     const int tid = static_cast<int>(threadIdx.x);
     const int nchunk = K >> 3;
     if constexpr (IMG_GS != 0) {
+        const size_t at = image_at(col, K);
+        img += at / sizeof(uint2);
+        fac += at / sizeof(float2);
+        us += at / sizeof(float);
         if (col >= ncols) {
             const float z[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
             for (int base = 0; base < nchunk; base += kNormThreads)  // uniform per workgroup
-                image_store8<IMG_GS>(z, base + tid, col, base + tid < nchunk, img, fac, us);
+                image_store8<IMG_GS>(z, base + tid, col % kImageCols, base + tid < nchunk, img, fac, us);
             return;
         }
     }
     const size_t c = static_cast<size_t>(col);
     float4* h = reinterpret_cast<float4*>(H + c * K);
     const float4* d = D ? reinterpret_cast<const float4*>(D + c * K) : nullptr;
-    float4* x = reinterpret_cast<float4*>(X + c * K);
+    float4* x = X ? reinterpret_cast<float4*>(X + c * K) : nullptr;
     const float4* w4 = reinterpret_cast<const float4*>(w);
     float ss = 0.0f;
     for (int ch = tid; ch < nchunk; ch += kNormThreads) {
@@ -932,11 +946,11 @@ __global__ __launch_bounds__(kNormThreads) void verify_add_norm_kernel(float* __
         const float v[8] = {(a.x * inv_rms) * wa.x, (a.y * inv_rms) * wa.y, (a.z * inv_rms) * wa.z,
                             (a.w * inv_rms) * wa.w, (b.x * inv_rms) * wb.x, (b.y * inv_rms) * wb.y,
                             (b.z * inv_rms) * wb.z, (b.w * inv_rms) * wb.w};
-        if (ch < nchunk) {
+        if (x && ch < nchunk) {
             x[2 * ch] = make_float4(v[0], v[1], v[2], v[3]);
             x[2 * ch + 1] = make_float4(v[4], v[5], v[6], v[7]);
         }
-        if constexpr (IMG_GS != 0) image_store8<IMG_GS>(v, ch, col, ch < nchunk, img, fac, us);
+        if constexpr (IMG_GS != 0) image_store8<IMG_GS>(v, ch, col % kImageCols, ch < nchunk, img, fac, us);
     }
 }
 
@@ -1084,8 +1098,8 @@ __global__ __launch_bounds__(kAttnThreads) void verify_attn_partial_kernel(
 // (swiglu_inplace, unified_engine.cpp:803-857; the decode prologue's formula).
 // S[c] = swiglu(GU[c][0:ffn], GU[c][ffn:2ffn]), one 8-element chunk per
 // thread (grid: ceil(ffn / 2048) x columns).  IMG_GS: also the down GEMV's
-// int8 image of S (image_store8), with zero image columns for c >= ncols (the
-// grid then covers kImageCols columns).
+// int8 image of S (image_store8; column c's image is c / kImageCols), with
+// zero image columns for c >= ncols; S may be null then.
 template <int IMG_GS>
 __global__ __launch_bounds__(256) void verify_swiglu_kernel(const float* __restrict__ GU, float* __restrict__ S,
                                                             int ffn, float thr, int ncols, uint2* __restrict__ img,
@@ -1103,13 +1117,19 @@ __global__ __launch_bounds__(256) void verify_swiglu_kernel(const float* __restr
         const float* g = GU + c * 2 * ffn + 8 * cc;
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = swiglu_ref(g[e], g[ffn + e], thr);
-        if (ch < nchunk) {
+        if (S && ch < nchunk) {
             float4* sp = reinterpret_cast<float4*>(S + c * ffn + 8 * ch);
             sp[0] = make_float4(v[0], v[1], v[2], v[3]);
             sp[1] = make_float4(v[4], v[5], v[6], v[7]);
         }
     }
-    if constexpr (IMG_GS != 0) image_store8<IMG_GS>(v, ch, col, ch < nchunk, img, fac, us);
+    if constexpr (IMG_GS != 0) {
+        const size_t at = image_at(col, ffn);
+        img += at / sizeof(uint2);
+        fac += at / sizeof(float2);
+        us += at / sizeof(float);
+        image_store8<IMG_GS>(v, ch, col % kImageCols, ch < nchunk, img, fac, us);
+    }
 }
 
 // keys[c] = max over rows of argmax_key(logits[c][row], row): the largest
@@ -1160,6 +1180,222 @@ __global__ void verify_tokens_kernel(const unsigned long long* __restrict__ keys
     if (c < n) next[c] = static_cast<int>(0xFFFFFFFFu - static_cast<uint32_t>(keys[c]));
 }
 
+// ----------------------------------------------------------------- prefill
+// A prompt chunk of n tokens at positions first .. first + n - 1, every
+// column with the single-token step's arithmetic: what bounds a prompt is the
+// fp32 steps of the projections (preq2_gemm_exact) and of the attention, so
+// each is done over all of the chunk's columns in one launch, and nothing is
+// computed that the prompt does not leave behind (no logits but the last
+// token's; the last layer past its K/V rows only for the last token).
+
+// Per column (blockIdx.y) and head, 16 lanes of 8 dims: the query heads
+// rotated to Q[c][n_heads * 128], the rotated key and the value into the
+// cache row of position first + c, exactly as the step's attention does it.
+template <bool Q8>
+__global__ __launch_bounds__(256) void prefill_rope_kv_kernel(const float* __restrict__ QKV, KvCache kv,
+                                                              const float* __restrict__ rope_cos,
+                                                              const float* __restrict__ rope_sin,
+                                                              float* __restrict__ Q, int first, int n_heads, int n_kv,
+                                                              int max_seq, int rot_half) {
+    const int c = static_cast<int>(blockIdx.y);
+    const int e = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    const int head = e >> 4;  // query heads, then key heads, then value heads
+    const int dc = e & 15;
+    if (head >= n_heads + 2 * n_kv) return;
+    const int pos = first + c;
+    const float* src = QKV + (static_cast<size_t>(c) * (n_heads + 2 * n_kv) + head) * kHeadDim;
+    float r[8];
+    if (head < n_heads + n_kv) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) r[k] = rope_dim(src, 8 * dc + k, pos, rot_half, rope_cos, rope_sin);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) r[k] = src[8 * dc + k];
+    }
+    if (head < n_heads) {
+        float4* dst = reinterpret_cast<float4*>(Q + (static_cast<size_t>(c) * n_heads + head) * kHeadDim + 8 * dc);
+        dst[0] = make_float4(r[0], r[1], r[2], r[3]);
+        dst[1] = make_float4(r[4], r[5], r[6], r[7]);
+        return;
+    }
+    const bool key = head < n_heads + n_kv;
+    const int kvh = head - n_heads - (key ? 0 : n_kv);
+    const size_t row = static_cast<size_t>(kvh) * max_seq + pos;
+    const uint4 p = kv_pack8<Q8>(r);
+    void* base = key ? kv.k : kv.v;
+    if constexpr (Q8) {
+        *reinterpret_cast<uint2*>(static_cast<int8_t*>(base) + row * kHeadDim + 8 * dc) = make_uint2(p.x, p.y);
+        if ((dc & 7) == 0) (key ? kv.ks : kv.vs)[row * 2 + (dc >> 3)] = __uint_as_float(p.z);
+    } else {
+        *reinterpret_cast<uint4*>(static_cast<uint16_t*>(base) + row * kHeadDim + 8 * dc) = p;
+    }
+}
+
+// Attention partials of the columns [blockIdx.z * cpw, + cpw) below n for KV
+// head blockIdx.y and split blockIdx.x: attn_decode_kernel's arithmetic (same
+// tiles of 4 * WAVES * KIT positions, tps of them a split, same lanes, same
+// merge), with every K/V row read from the cache.  The instruction rate of
+// the vector unit bounds it (about 650 instructions per wave, column and
+// tile), so a workgroup converts a tile's K/V rows to fp32 once for all of its
+// columns when a split is one tile (positions below 2048); with more tiles a
+// column reads them in turn.  The merge's LDS area alternates between
+// columns, which leaves two barriers per column.
+template <int G, bool Q8, int WAVES, int KIT>
+__global__ __launch_bounds__(WAVES * kWave) void prefill_attn_kernel(const float* __restrict__ Q, KvCache kv,
+                                                                    float* __restrict__ part, int first, int c_begin,
+                                                                    int c_end, int cpw, int n_heads, int max_seq,
+                                                                    int nsplit, int tps) {
+#pragma clang fp contract(off)  // rounds as attn_split_core does
+    constexpr int kThreads = WAVES * kWave;
+    constexpr int kStep = 4 * WAVES;
+    constexpr int kTile = kStep * KIT;
+    constexpr int NG = kThreads / 16;
+    __shared__ float gml[2][NG][G][2];
+    __shared__ __align__(16) float gacc[2][NG][G][kHeadDim];
+    __shared__ float ge[2][G][NG];
+    const int s = static_cast<int>(blockIdx.x);
+    const int kvh = static_cast<int>(blockIdx.y);
+    // the columns with the most splits first
+    const int c0 = c_begin + static_cast<int>(gridDim.z - 1 - blockIdx.z) * cpw;
+    const int c1 = min(c0 + cpw, c_end);
+    const int p0 = s * tps * kTile;
+    const int cb = max(c0, p0 - first);  // the first column that sees position p0
+    if (cb >= c1) return;
+    const int tid = static_cast<int>(threadIdx.x);
+    const int lane = tid & (kWave - 1);
+    const int wave = tid >> 6;
+    const int pg = lane >> 4;
+    const int dc = lane & 15;
+    const size_t row0 = static_cast<size_t>(kvh) * max_seq;
+    const int p_last = first + c1 - 1;  // rows past it are not read
+    const float inv_sqrt_d = 1.0f / sqrtf(static_cast<float>(kHeadDim));
+
+    float k8[KIT][8], v8[KIT][8];
+    auto load_tile = [&](int t0) {
+        uint4 kr[KIT], vr[KIT];
+#pragma unroll
+        for (int it = 0; it < KIT; ++it) {
+            const size_t row = row0 + min(t0 + wave * 4 + pg + kStep * it, p_last);
+            kr[it] = kv_load8<Q8>(kv.k, kv.ks, row, dc);
+            vr[it] = kv_load8<Q8>(kv.v, kv.vs, row, dc);
+        }
+#pragma unroll
+        for (int it = 0; it < KIT; ++it) {
+            kv_unpack8<Q8>(kr[it], k8[it]);
+            kv_unpack8<Q8>(vr[it], v8[it]);
+        }
+    };
+    float qr[G][8], qn[G][8];
+    auto load_q = [&](int c, float (&q)[G][8]) {
+        const float4* src =
+            reinterpret_cast<const float4*>(Q + (static_cast<size_t>(c) * n_heads + kvh * G) * kHeadDim + 8 * dc);
+#pragma unroll
+        for (int hh = 0; hh < G; ++hh) {
+            const float4 a = src[hh * (kHeadDim / 4)], b = src[hh * (kHeadDim / 4) + 1];
+            q[hh][0] = a.x; q[hh][1] = a.y; q[hh][2] = a.z; q[hh][3] = a.w;
+            q[hh][4] = b.x; q[hh][5] = b.y; q[hh][6] = b.z; q[hh][7] = b.w;
+        }
+    };
+    load_q(cb, qn);
+    if (tps == 1) load_tile(p0);
+    int parity = 0;
+    for (int c = cb; c < c1; ++c) {  // uniform per workgroup
+        const int p1 = min(p0 + tps * kTile, first + c + 1);
+#pragma unroll
+        for (int hh = 0; hh < G; ++hh)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qr[hh][e] = qn[hh][e];
+        load_q(min(c + 1, c1 - 1), qn);
+        float m[G], l[G], acc[G][8];
+#pragma unroll
+        for (int hh = 0; hh < G; ++hh) {
+            m[hh] = -INFINITY;
+            l[hh] = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[hh][e] = 0.0f;
+        }
+        // MASKED: the tile reaches past the column's position, whose rows
+        // must not touch the sums (not even as 0 * inf)
+        auto process = [&](auto masked, int t) __attribute__((always_inline)) {
+            constexpr bool MASKED = decltype(masked)::value;
+            float sr[KIT][G];
+#pragma unroll
+            for (int it = 0; it < KIT; ++it) {
+                const int p = t + wave * 4 + pg + kStep * it;
+#pragma unroll
+                for (int hh = 0; hh < G; ++hh) {
+                    float d = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) d = fmaf(qr[hh][e], k8[it][e], d);
+                    d += dpp<kDppQuadXor1>(d);  // sum over the 16 lanes of the position
+                    d += dpp<kDppQuadXor2>(d);
+                    d += dpp<kDppRowRor4>(d);
+                    d += dpp<kDppRowRor8>(d);
+                    sr[it][hh] = !MASKED || p < p1 ? d * inv_sqrt_d : -INFINITY;
+                }
+            }
+#pragma unroll
+            for (int hh = 0; hh < G; ++hh) {
+                float v = sr[0][hh];
+#pragma unroll
+                for (int it = 1; it < KIT; ++it) v = fmaxf(v, sr[it][hh]);
+                if (t == p0) {  // uniform
+                    m[hh] = v;
+                } else {
+                    const float mn = fmaxf(m[hh], v);
+                    const float rs = m[hh] == -INFINITY ? 0.0f : expf(m[hh] - mn);
+                    m[hh] = mn;
+                    l[hh] *= rs;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[hh][e] *= rs;
+                }
+            }
+#pragma unroll
+            for (int it = 0; it < KIT; ++it) {
+                const int p = t + wave * 4 + pg + kStep * it;
+                const bool in = !MASKED || p < p1;
+#pragma unroll
+                for (int hh = 0; hh < G; ++hh) {
+                    const float w = in ? expf(sr[it][hh] - m[hh]) : 0.0f;
+                    l[hh] += w;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[hh][e] = in ? fmaf(w, v8[it][e], acc[hh][e]) : acc[hh][e];
+                }
+            }
+        };
+        for (int t = p0; t < p1; t += kTile) {
+            if (tps != 1) load_tile(t);
+            if (t + kTile <= p1) process(std::false_type{}, t);
+            else process(std::true_type{}, t);
+        }
+        merge_position_groups<G, kThreads>(
+            m, l, acc, gml[parity], gacc[parity], ge[parity],
+            part + ((static_cast<size_t>(c) * n_heads + kvh * G) * nsplit + s) * kPartStride,
+            static_cast<size_t>(nsplit) * kPartStride);
+        parity ^= 1;
+    }
+}
+
+// *pos = the chunk's first position (the combine reads it there), *key = 0,
+// *last_pos = the last column's.
+__global__ void prefill_begin_kernel(int* __restrict__ pos, int first, int* __restrict__ last_pos, int last,
+                                     unsigned long long* __restrict__ key) {
+    if (threadIdx.x == 0) {
+        *pos = first;
+        *last_pos = last;
+        *key = 0ull;
+    }
+}
+
+// *token = the argmax row of the last column (logits computed), *pos = next.
+__global__ void prefill_finish_kernel(const unsigned long long* __restrict__ key, int* __restrict__ token,
+                                      int* __restrict__ pos, int next) {
+    if (threadIdx.x == 0) {
+        if (key) *token = static_cast<int>(0xFFFFFFFFu - static_cast<uint32_t>(*key));
+        *pos = next;
+    }
+}
+
 // Zero the cache rows [from, max_seq) of every KV head (zero_kv_from,
 // unified_engine.cpp:1263-1283), 16-byte stores.
 __global__ __launch_bounds__(256) void kv_zero_kernel(uint4* __restrict__ k, uint4* __restrict__ v, int n_kv,
@@ -1202,6 +1438,87 @@ template <int G, bool Q8>
 struct VerifyAttnK {
     static auto fn() { return verify_attn_partial_kernel<G, Q8>; }
 };
+
+template <int G, bool Q8>
+struct PrefillAttnK {  // positions below kDeepFrom
+    static auto fn() { return prefill_attn_kernel<G, Q8, kLongForm.waves, kLongForm.tile / (4 * kLongForm.waves)>; }
+};
+template <int G, bool Q8>
+struct PrefillDeepAttnK {
+    static auto fn() { return prefill_attn_kernel<G, Q8, kDeepForm.waves, kDeepForm.tile / (4 * kDeepForm.waves)>; }
+};
+
+// Columns of a chunk: its buffers stay below 250 MB at the largest widths,
+// and from a few hundred columns a longer chunk gains nothing.
+constexpr int kMaxPrefillTokens = 512;
+
+// Work buffer layout of a prefill chunk of up to n tokens (offsets in floats).
+struct PrefillWork {
+    size_t H, QKV, Q, part, O, GU, img, att, h1, gu1, down1, key, last_pos, total;
+    int nsplit;
+};
+
+PrefillWork prefill_work(const asdsl_decode_model& m, int n) {
+    PrefillWork w{};
+    size_t at = 0;
+    auto take = [&](size_t cnt) {
+        const size_t here = at;
+        at += align64(cnt);
+        return here;
+    };
+    const size_t N = static_cast<size_t>(n);
+    const int qkv_dim = (m.n_heads + 2 * m.n_kv_heads) * m.head_dim;
+    const int wide = m.hidden > m.ffn ? m.hidden : m.ffn;
+    w.nsplit = attn_max_splits(m.max_seq, kLongForm);
+    w.H = take(N * m.hidden);
+    w.QKV = take(N * qkv_dim);
+    w.Q = take(N * m.n_heads * m.head_dim);
+    w.part = take(N * m.n_heads * w.nsplit * kPartStride);
+    w.O = take(N * m.hidden);
+    w.GU = take(N * 2 * m.ffn);
+    w.img = take((N + kImageCols - 1) / kImageCols * image_bytes(wide) / sizeof(float));
+    // the last token's rows past the last layer's attention
+    w.att = take(static_cast<size_t>(m.n_heads) * m.head_dim);
+    w.h1 = take(m.hidden);
+    w.gu1 = take(2 * static_cast<size_t>(m.ffn));
+    w.down1 = take(m.hidden);
+    w.key = take(2);
+    w.last_pos = take(1);
+    w.total = at;
+    return w;
+}
+
+// Partials of columns [c_begin, c_end) of a chunk whose column c is at
+// position first + c.
+asdsl_status launch_prefill_attention(const float* Q, const KvCache& kv, bool q8, float* part, int first, int c_begin,
+                                      int c_end, int n_heads, int n_kv, int max_seq, int nsplit, int cus,
+                                      hipStream_t s) {
+    // positions of one form and one split size per launch: below 2048 one
+    // tile a split, then one tile more from every 2048 positions
+    for (int c0 = c_begin; c0 < c_end;) {
+        const int pos = first + c0;
+        const bool deep = pos >= kDeepFrom;
+        const FoldForm& f = deep ? kDeepForm : kLongForm;
+        const int tps = attn_fold_tps(pos, f.tile, f.max_splits);
+        const int span = f.tile * f.max_splits;
+        const int c1 = min(c_end, (pos / span + 1) * span - first);
+        const int splits = attn_fold_splits(first + c1 - 1, f.tile, f.max_splits);
+        // Columns per workgroup: up to 16 share a tile's rows, fewer while
+        // that would leave less than two workgroups per compute unit.
+        int cpw = 16;
+        while (cpw > 1 && static_cast<long long>(splits) * n_kv * ((c1 - c0 + cpw - 1) / cpw) < 2LL * cus) cpw >>= 1;
+        const dim3 grid(splits, n_kv, (c1 - c0 + cpw - 1) / cpw);
+        auto go = [&](auto kern) {
+            return launch("prefill_attn_kernel", kern, grid, dim3(f.waves * kWave), 0, s, Q, kv, part, first, c0, c1,
+                          cpw, n_heads, max_seq, nsplit, tps);
+        };
+        const asdsl_status st = deep ? with_attn_kernel<PrefillDeepAttnK>(n_heads / n_kv, q8, go)
+                                     : with_attn_kernel<PrefillAttnK>(n_heads / n_kv, q8, go);
+        if (st != ASDSL_OK) return st;
+        c0 = c1;
+    }
+    return ASDSL_OK;
+}
 
 // Work buffer layout of a verify pass of up to n tokens (offsets in floats).
 struct VerifyWork {
@@ -1601,6 +1918,141 @@ extern "C" asdsl_status asdsl_decode_verify(const asdsl_decode_model* model, con
     if (st != ASDSL_OK) return st;
     return launch("verify_tokens_kernel", verify_tokens_kernel, dim3(1), dim3(kWave), 0, s,
                   static_cast<const unsigned long long*>(keys), next_tokens, n);
+}
+
+extern "C" size_t asdsl_decode_prefill_work_bytes(const asdsl_decode_model* model, int max_tokens) {
+    if (check_model(model) != ASDSL_OK || max_tokens < 1 || max_tokens > kMaxPrefillTokens) return 0;
+    return prefill_work(*model, max_tokens).total * sizeof(float);
+}
+
+extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, const int* tokens, int n_tokens,
+                                             int start_pos, int* token, int* pos, float* logits, void* work,
+                                             asdsl_stream_t stream) {
+    const asdsl_status cs = check_model(model);
+    if (cs != ASDSL_OK) return cs;
+    ASDSL_CHECK_ARG(tokens && token && pos && work, "decode_prefill: null pointer");
+    ASDSL_CHECK_ARG(n_tokens >= 1 && n_tokens <= kMaxPrefillTokens, "decode_prefill: n_tokens must be in [1, %d]",
+                    kMaxPrefillTokens);
+    const asdsl_decode_model& m = *model;
+    ASDSL_CHECK_ARG(start_pos >= 0 && start_pos <= m.max_seq - n_tokens,
+                    "decode_prefill: positions out of the cache's range");
+    ASDSL_CHECK_ARG(reinterpret_cast<uintptr_t>(work) % 256 == 0, "decode_prefill: work must be 256-byte aligned");
+    // the factored norm (ASDSL_HIP_NORM_FACTORED) is the step's other
+    // arithmetic, which the chunk's norm kernel does not have
+    if (preq2_norm_factored()) {
+        set_error("decode_prefill: not with the factored norm");
+        return ASDSL_ERR_UNSUPPORTED;
+    }
+    ASDSL_CU_COUNT(cus);
+    const int n = n_tokens;
+    const PrefillWork w = prefill_work(m, n);
+    float* base = static_cast<float*>(work);
+    float* H = base + w.H;
+    float* QKV = base + w.QKV;
+    float* Q = base + w.Q;
+    float* part = base + w.part;
+    float* O = base + w.O;
+    float* GU = base + w.GU;
+    auto* key = reinterpret_cast<unsigned long long*>(base + w.key);
+    int* last_pos = reinterpret_cast<int*>(base + w.last_pos);
+    void* image = base + w.img;
+    auto* img = reinterpret_cast<uint2*>(base + w.img);
+    hipStream_t s = as_hip(stream);
+    const int qkv_dim = (m.n_heads + 2 * m.n_kv_heads) * m.head_dim;
+    const int q_dim = m.n_heads * m.head_dim;
+    const bool q8 = m.kv_format == ASDSL_KV_INT8;
+    auto fac_of = [&](int K) { return reinterpret_cast<float2*>(static_cast<uint8_t*>(image) + image_fac_offset(K)); };
+    auto us_of = [&](int K) { return reinterpret_cast<float*>(static_cast<uint8_t*>(image) + image_us_offset(K)); };
+    // up to one image the kernels that split K over waves, where they apply
+    auto gemm = [&](const uint8_t* meta, const uint8_t* quant, float* Y, int M, int K, int gs) -> asdsl_status {
+        return n <= kImageCols && preq2_batch_exact_mfma_applies(M, K, gs, n)
+                   ? preq2_batch_exact_mfma_image(meta, quant, image, Y, M, K, gs, n, stream)
+                   : preq2_gemm_exact(meta, quant, image, Y, M, K, gs, n, stream);
+    };
+    auto norm_then_gemm = [&](const float* D, const float* nw, const uint8_t* meta, const uint8_t* quant, float* Y,
+                              int M, int gs) -> asdsl_status {
+        const int K = m.hidden;
+        const asdsl_status r = launch("verify_add_norm_kernel",
+                                      gs == 32 ? verify_add_norm_kernel<32> : verify_add_norm_kernel<128>, dim3(n),
+                                      dim3(kNormThreads), 0, s, H, D, nw, static_cast<float*>(nullptr), K, m.rms_eps,
+                                      n, img, fac_of(K), us_of(K), static_cast<float*>(nullptr));
+        return r != ASDSL_OK ? r : gemm(meta, quant, Y, M, K, gs);
+    };
+
+    asdsl_status st = launch("prefill_begin_kernel", prefill_begin_kernel, dim3(1), dim3(kWave), 0, s, pos, start_pos,
+                             last_pos, start_pos + n - 1, key);
+    if (st != ASDSL_OK) return st;
+    st = launch("verify_embed_kernel", verify_embed_kernel, dim3((m.hidden + 1023) / 1024, n), dim3(256), 0, s, m.embed,
+                tokens, H, m.hidden, m.vocab, static_cast<unsigned long long*>(nullptr));
+    if (st != ASDSL_OK) return st;
+    const float* pending = nullptr;
+    for (int l = 0; l < m.n_layers; ++l) {
+        const asdsl_decode_layer& L = m.layers[l];
+        const bool last = l + 1 == m.n_layers;
+        st = norm_then_gemm(pending, L.rms_att, L.qkv_meta, L.qkv_quant, QKV, qkv_dim, m.gs_attn);
+        if (st != ASDSL_OK) return st;
+        const KvCache kv{L.k_cache, L.v_cache, L.k_scale, L.v_scale};
+        const dim3 rgrid(((m.n_heads + 2 * m.n_kv_heads) * 16 + 255) / 256, n);
+        st = launch("prefill_rope_kv_kernel", q8 ? prefill_rope_kv_kernel<true> : prefill_rope_kv_kernel<false>, rgrid,
+                    dim3(256), 0, s, static_cast<const float*>(QKV), kv, m.rope_cos, m.rope_sin, Q, start_pos,
+                    m.n_heads, m.n_kv_heads, m.max_seq, m.rotary_dim / 2);
+        if (st != ASDSL_OK) return st;
+        if (last && !logits) break;  // the K/V rows are all that the chunk leaves
+        st = launch_prefill_attention(Q, kv, q8, part, start_pos, last ? n - 1 : 0, n, m.n_heads, m.n_kv_heads,
+                                      m.max_seq, w.nsplit, cus, s);
+        if (st != ASDSL_OK) return st;
+        const dim3 cthreads(combine_threads(w.nsplit));
+        if (last) {  // only the last token's: the single-token step's launches
+            float* att = base + w.att;
+            float* h1 = base + w.h1;
+            float* gu1 = base + w.gu1;
+            float* down1 = base + w.down1;
+            const size_t col = static_cast<size_t>(n - 1);
+            const float* h = H + col * m.hidden;
+            st = launch("attn_combine_kernel", attn_combine_kernel<0>, dim3(m.n_heads), cthreads, 0, s,
+                        static_cast<const float*>(part) + col * m.n_heads * w.nsplit * kPartStride,
+                        static_cast<const int*>(last_pos), att, w.nsplit, m.max_seq, m.max_seq, 0, 1, kLongForm.tile,
+                        kLongForm.max_splits, static_cast<uint2*>(nullptr), static_cast<float2*>(nullptr),
+                        static_cast<float*>(nullptr));
+            if (st != ASDSL_OK) return st;
+            st = asdsl_gemv_preq2_fused(L.o_meta, L.o_quant, att, O, m.hidden, q_dim, m.gs_attn, stream);
+            if (st != ASDSL_OK) return st;
+            st = asdsl_gemv_preq2_rmsnorm_swiglu(L.gu_meta, L.gu_quant, h, O, L.rms_ffn, h1, gu1, m.ffn, m.hidden,
+                                                 m.gs_ffn, m.rms_eps, L.fatrelu_threshold, stream);
+            if (st == ASDSL_OK) {
+                st = asdsl_gemv_preq2_fused(L.down_meta, L.down_quant, gu1, down1, m.hidden, m.ffn, m.gs_ffn, stream);
+            } else if (st == ASDSL_ERR_UNSUPPORTED) {
+                st = asdsl_gemv_preq2_rmsnorm(L.gu_meta, L.gu_quant, h, O, L.rms_ffn, h1, gu1, 2 * m.ffn, m.hidden,
+                                              m.gs_ffn, m.rms_eps, nullptr, stream);
+                if (st != ASDSL_OK) return st;
+                st = asdsl_gemv_preq2_swiglu(L.down_meta, L.down_quant, gu1, down1, m.hidden, m.ffn, m.gs_ffn,
+                                             L.fatrelu_threshold, stream);
+            }
+            if (st != ASDSL_OK) return st;
+            st = asdsl_gemv_preq2_rmsnorm(m.lm_meta, m.lm_quant, h1, down1, m.rms_out, nullptr, logits, m.vocab,
+                                          m.hidden, m.gs_lm, m.rms_eps, key, stream);
+            if (st != ASDSL_OK) return st;
+            break;
+        }
+        st = launch("attn_combine_kernel", m.gs_attn == 32 ? attn_combine_kernel<32> : attn_combine_kernel<128>,
+                    dim3(m.n_heads, n), cthreads, 0, s, static_cast<const float*>(part), static_cast<const int*>(pos),
+                    static_cast<float*>(nullptr), w.nsplit, m.max_seq, m.max_seq, 0, n, kLongForm.tile,
+                    kLongForm.max_splits, img, fac_of(q_dim), us_of(q_dim));
+        if (st != ASDSL_OK) return st;
+        st = gemm(L.o_meta, L.o_quant, O, m.hidden, q_dim, m.gs_attn);
+        if (st != ASDSL_OK) return st;
+        st = norm_then_gemm(O, L.rms_ffn, L.gu_meta, L.gu_quant, GU, 2 * m.ffn, m.gs_ffn);
+        if (st != ASDSL_OK) return st;
+        st = launch("verify_swiglu_kernel", m.gs_ffn == 32 ? verify_swiglu_kernel<32> : verify_swiglu_kernel<128>,
+                    dim3((m.ffn / 8 + 255) / 256, n), dim3(256), 0, s, static_cast<const float*>(GU),
+                    static_cast<float*>(nullptr), m.ffn, L.fatrelu_threshold, n, img, fac_of(m.ffn), us_of(m.ffn));
+        if (st != ASDSL_OK) return st;
+        st = gemm(L.down_meta, L.down_quant, O, m.hidden, m.ffn, m.gs_ffn);
+        if (st != ASDSL_OK) return st;
+        pending = O;
+    }
+    return launch("prefill_finish_kernel", prefill_finish_kernel, dim3(1), dim3(kWave), 0, s,
+                  static_cast<const unsigned long long*>(logits ? key : nullptr), token, pos, start_pos + n);
 }
 
 extern "C" asdsl_status asdsl_kv_zero_from(uint16_t* k_cache, uint16_t* v_cache, int n_kv_heads, int head_dim,

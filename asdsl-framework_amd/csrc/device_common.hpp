@@ -313,6 +313,13 @@ __host__ __device__ constexpr size_t image_fac_offset(int K) { return static_cas
 __host__ __device__ constexpr size_t image_us_offset(int K) { return static_cast<size_t>(K) * 20; }
 __host__ __device__ constexpr size_t image_bytes(int K) { return static_cast<size_t>(K) * 22; }
 
+// A pass of more than kImageCols columns keeps one image per 16 of them,
+// image_bytes(K) apart: the byte offset of column `col`'s image (its column in
+// it is col % kImageCols).
+__device__ __forceinline__ size_t image_at(int col, int K) {
+    return static_cast<size_t>(col / kImageCols) * image_bytes(K);
+}
+
 // Decode-step elementwise helpers shared by the fused GEMV prologues and the
 // batched verify pass, so both compute identical values.
 

@@ -590,6 +590,23 @@ size_t asdsl_decode_verify_work_bytes(const asdsl_decode_model* model, int max_t
 asdsl_status asdsl_decode_verify(const asdsl_decode_model* model, const int* tokens, int n_tokens, const int* pos,
                                  float* logits, int* next_tokens, void* work, asdsl_stream_t stream);
 
+/* Bytes of device work buffer asdsl_decode_prefill needs for up to max_tokens
+ * tokens (1..512); 0 for an invalid model or count. */
+size_t asdsl_decode_prefill_work_bytes(const asdsl_decode_model* model, int max_tokens);
+
+/* Queues one chunk of a prompt: tokens[0..n) (device) at positions start_pos
+ * .. start_pos + n - 1, every column with the single-token step's arithmetic.
+ * Writes the chunk's K/V rows; with logits (device [vocab], may be null) also
+ * the last token's logits and *token = their greedy argmax; *pos = start_pos +
+ * n (device ints; *pos is used as scratch meanwhile).  What it writes is what
+ * asdsl_decode_token on each token in turn leaves, bit for bit.  1 <= n <=
+ * 512, start_pos + n <= max_seq; work: asdsl_decode_prefill_work_bytes(model,
+ * >= n) bytes, 256-byte aligned.  ASDSL_ERR_UNSUPPORTED (nothing queued) under
+ * ASDSL_HIP_NORM_FACTORED.  The reference feeds a prompt one forward_token
+ * per token (asdsl/kernels/native/unified_engine.cpp:1339-1688). */
+asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, const int* tokens, int n_tokens, int start_pos,
+                                  int* token, int* pos, float* logits, void* work, asdsl_stream_t stream);
+
 /* The int8 cache's form of asdsl_kv_zero_from: codes 0 and scales 1.0 in rows
  * [from_pos, max_seq), as zero_kv_from leaves them
  * (asdsl/kernels/native/unified_engine.cpp:1263-1283). */

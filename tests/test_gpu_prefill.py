@@ -1,0 +1,79 @@
+"""HIP parity for the prompt path (asdsl_decode_prefill): a prompt run in
+chunks leaves what forward_token on each of its tokens leaves (the decode step
+itself is checked against the oracle in test_gpu_decode*.py).  Tolerance: none.
+The chunk repeats the step's arithmetic operation for operation, so every bit
+of the K/V rows and the logits agrees."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(eng):
+    names = ("k_cache", "v_cache") + (("k_scale", "v_scale") if eng.kv_int8 else ())
+    return (eng.logits.clone(), eng.next_token(), int(eng.pos.item()), eng._host_pos, eng.get_kv_seq_len(),
+            [L[n].clone() for L in eng.layers for n in names])
+
+
+def _compare(cfg, plens, seed=5):
+    import torch
+    from asdsl.engine import DecodeEngine
+
+    eng = DecodeEngine.synthetic(cfg, seed=seed, fatrelu_threshold=0.0)
+    rng = np.random.default_rng(seed)
+    prompt = [int(t) for t in rng.integers(0, cfg.vocab, max(plens))]
+    for n in plens:
+        eng.reset_session()
+        eng.prefill(prompt[:n])
+        got = _state(eng)
+        eng.reset_session()
+        for i, t in enumerate(prompt[:n]):
+            eng.forward_token(t, i)
+        want = _state(eng)
+        assert got[1:5] == want[1:5] == (want[1], n, n, n), n
+        for a, b in zip(got[5], want[5]):
+            assert torch.equal(a, b), n
+        assert torch.equal(got[0], want[0]), n
+
+
+# 4: the smallest chunk; 16 and 17: one column block and the first of two; 64
+# and 65: a workgroup's 4 blocks and a tile of positions, and one past; 512 and
+# 530: a whole chunk, and a second one
+@pytest.mark.parametrize("kv", ["fp16", "int8"])
+def test_prompt_lengths(gpu, kv):
+    from asdsl.engine import DecodeConfig
+
+    _compare(DecodeConfig(n_layers=2, vocab=4096, max_seq=576, kv_format=kv), (4, 16, 17, 64, 65, 197, 512, 530))
+
+
+# group sizes in both places, query heads per KV head 1, 2 and 4, and in_features
+# whose K split masks units (3712 = 29 groups of 128) or leaves a class of
+# groups empty (1152: 9 groups of 128)
+@pytest.mark.parametrize("heads,kv_heads,ffn,gs_attn,gs_ffn", [
+    (8, 4, 3712, 32, 128), (8, 8, 1152, 128, 32), (16, 4, 8192, 32, 32), (9, 3, 2944, 128, 128)])
+def test_shapes(gpu, heads, kv_heads, ffn, gs_attn, gs_ffn):
+    from asdsl.engine import DecodeConfig
+
+    _compare(DecodeConfig(hidden=128 * heads, n_heads=heads, n_kv_heads=kv_heads, ffn=ffn, vocab=1003, n_layers=3,
+                          max_seq=160, gs_attn=gs_attn, gs_ffn=gs_ffn), (18, 77, 150))
+
+
+# past 2048 positions a split holds two tiles, past 4096 three
+@pytest.mark.parametrize("kv,plen", [("fp16", 2130), ("int8", 4101)])
+def test_deep_positions(gpu, kv, plen):
+    from asdsl.engine import DecodeConfig
+
+    _compare(DecodeConfig(hidden=1024, n_heads=8, n_kv_heads=4, ffn=1536, vocab=2048, n_layers=2, max_seq=plen + 3,
+                          kv_format=kv), (plen,))
+
+
+def test_refused(gpu):
+    from asdsl.engine import DecodeConfig, DecodeEngine
+
+    eng = DecodeEngine.synthetic(DecodeConfig(hidden=1024, n_heads=8, n_kv_heads=4, ffn=1536, vocab=2048, n_layers=1,
+                                              max_seq=64), seed=1)
+    with pytest.raises(ValueError, match="vocab"):
+        eng.prefill([1, 2, 3, 4, 2048])
+    with pytest.raises(ValueError, match="range"):
+        eng.prefill([1] * 65)
