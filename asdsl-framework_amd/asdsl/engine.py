@@ -477,8 +477,8 @@ class DecodeEngine:
     # it on the step's deep attention form splits differently.
     EXACT_BATCH_LIMIT = 2048
 
-    # tokens of one prefill chunk
-    MAX_PREFILL_TOKENS = 512
+    # tokens of one prefill chunk at most (a prompt's chunks are of one size)
+    MAX_PREFILL_TOKENS = 1024
 
     def prefill(self, tokens) -> None:
         """The prompt tokens at positions 0, 1, ...: the K/V rows, the device
@@ -514,7 +514,9 @@ class DecodeEngine:
             raise ValueError("prefill: token_id out of vocab range")
         if len(toks) > c.max_seq:
             raise ValueError("prefill: positions out of kv-cache range")
-        most = min(len(toks), self.MAX_PREFILL_TOKENS)
+        chunks = -(-len(toks) // self.MAX_PREFILL_TOKENS)
+        chunk = min(-(-len(toks) // (16 * chunks)) * 16, self.MAX_PREFILL_TOKENS)
+        most = min(len(toks), chunk)
         if self._prefill_work is None or self._prefill_tokens < most:
             # grown in steps, so that prompts of rising length allocate a few times only
             most = min(max(most, 2 * self._prefill_tokens, 64), self.MAX_PREFILL_TOKENS)
@@ -525,8 +527,8 @@ class DecodeEngine:
             self._prefill_tokens = most
         ids = torch.tensor(toks, dtype=torch.int32).to(self.token.device)
         stream = _hip.stream_handle()
-        for pos in range(0, len(toks), self.MAX_PREFILL_TOKENS):
-            n = min(self.MAX_PREFILL_TOKENS, len(toks) - pos)
+        for pos in range(0, len(toks), chunk):
+            n = min(chunk, len(toks) - pos)
             last = pos + n == len(toks)
             _hip.check(_hip.LIB.asdsl_decode_prefill(ctypes.byref(self._model), _hip.ptr(ids[pos:]), n, pos,
                                                      _hip.ptr(self.token), _hip.ptr(self.pos),

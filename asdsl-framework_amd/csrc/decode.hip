@@ -297,7 +297,7 @@ __device__ __forceinline__ void kv_quantize_new(float (*kv_new)[kHeadDim], const
 // splits (chunks of kChunk loads issued together, a running (max, sum,
 // output) rescaled between chunks); with more than one group the runs are
 // merged in LDS in split order.  One group when the splits fit one chunk.
-// blockIdx.y = column c of a multi-token pass (position *pos_ptr + c; its
+// blockIdx.y = column c of a multi-token pass (position *pos_ptr + c0 + c; its
 // partials and output follow column c - 1's); the decode step runs one column.
 constexpr int kCombineGroups = 8;
 constexpr int kCombineThreads = kCombineGroups * kHeadDim;
@@ -314,11 +314,11 @@ inline int combine_threads(int max_ns) {
 
 // IMG_GS (32 or 128): the head's 128 outputs of column c are also quantized
 // into the o_proj batched GEMV's int8 image (image_store8, 16 chunks per
-// head; column c's image is c / kImageCols), and columns c >= ncols write
+// head, as column c0 + c of the pass), and columns at or past ncols write
 // that image's zero columns.  out may be null then.
 template <int IMG_GS>
 __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const float* __restrict__ part,
-                                                                      const int* __restrict__ pos_ptr,
+                                                                      const int* __restrict__ pos_ptr, int c0,
                                                                       float* __restrict__ out, int nsplit,
                                                                       int max_seq, int pos_limit, int fold, int ncols,
                                                                       int form_tile, int form_splits,
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const flo
     __shared__ float gml[kCombineGroups][2];
     __shared__ float go[kCombineGroups][kHeadDim];
     __shared__ float res_s[IMG_GS != 0 ? kHeadDim : 1];
-    const int col = static_cast<int>(blockIdx.y);
+    const int col = c0 + static_cast<int>(blockIdx.y);
     const int h = static_cast<int>(blockIdx.x);
     const int tid = static_cast<int>(threadIdx.x);
     const int d = tid % kHeadDim;
@@ -352,8 +352,8 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const flo
         return;
     }
     const int pos = *pos_ptr + col;
-    part += static_cast<size_t>(col) * gridDim.x * nsplit * kPartStride;
-    if (out) out += static_cast<size_t>(col) * gridDim.x * kHeadDim;
+    part += static_cast<size_t>(blockIdx.y) * gridDim.x * nsplit * kPartStride;
+    if (out) out += static_cast<size_t>(blockIdx.y) * gridDim.x * kHeadDim;
     if (pos < 0 || pos >= max_seq || pos >= pos_limit) {  // no partials were written (see attn_decode_kernel)
         if (g == 0 && out) out[static_cast<size_t>(h) * kHeadDim + d] = 0.0f;
         if (IMG_GS != 0 && tid < kHeadChunks) image_chunk(zeros);
@@ -764,7 +764,7 @@ asdsl_status launch_attention_decode(const float* qkv, const KvCache& kv, bool q
     if (st != ASDSL_OK || fold) return st;
     const StageScope stage("attention_combine");
     return launch("attn_combine_kernel", attn_combine_kernel<0>, dim3(n_heads), dim3(combine_threads(grid.x)), 0, s,
-                  static_cast<const float*>(work), pos, att, kMaxSplits, max_seq, limit, 0, 1, f.tile, f.max_splits,
+                  static_cast<const float*>(work), pos, 0, att, kMaxSplits, max_seq, limit, 0, 1, f.tile, f.max_splits,
                   static_cast<uint2*>(nullptr), static_cast<float2*>(nullptr), static_cast<float*>(nullptr));
 }
 
@@ -1235,11 +1235,14 @@ __global__ __launch_bounds__(256) void prefill_rope_kv_kernel(const float* __res
 // head blockIdx.y and split blockIdx.x: attn_decode_kernel's arithmetic (same
 // tiles of 4 * WAVES * KIT positions, tps of them a split, same lanes, same
 // merge), with every K/V row read from the cache.  The instruction rate of
-// the vector unit bounds it (about 650 instructions per wave, column and
-// tile), so a workgroup converts a tile's K/V rows to fp32 once for all of its
-// columns when a split is one tile (positions below 2048); with more tiles a
-// column reads them in turn.  The merge's LDS area alternates between
-// columns, which leaves two barriers per column.
+// the vector unit bounds it: 530 instructions per wave, column and tile at
+// three query heads, 70 % of the issue slots taken (154 us for 512 columns of
+// 24 heads from position 0).  So a workgroup converts a tile's K/V rows to
+// fp32 once for all of its columns when a split is one tile (positions below
+// 2048); with more tiles a column reads them in turn.  Forming each weight
+// once per quad instead of in every lane took 630 to 530 instructions.  The
+// merge's LDS area alternates between columns, which leaves two barriers per
+// column.
 template <int G, bool Q8, int WAVES, int KIT>
 __global__ __launch_bounds__(WAVES * kWave) void prefill_attn_kernel(const float* __restrict__ Q, KvCache kv,
                                                                     float* __restrict__ part, int first, int c_begin,
@@ -1350,17 +1353,35 @@ __global__ __launch_bounds__(WAVES * kWave) void prefill_attn_kernel(const float
                     for (int e = 0; e < 8; ++e) acc[hh][e] *= rs;
                 }
             }
+            // The four lanes of a quad hold the same scores, so lane j of
+            // each forms step j's weights and the others take them from it.
+            static_assert(KIT == 2 || KIT == 4, "a step per lane of a quad, or per two");
+            float we[G];
+            const int j = lane & (KIT - 1);
+            const bool in_j = !MASKED || t + wave * 4 + pg + kStep * j < p1;
 #pragma unroll
-            for (int it = 0; it < KIT; ++it) {
-                const int p = t + wave * 4 + pg + kStep * it;
-                const bool in = !MASKED || p < p1;
+            for (int hh = 0; hh < G; ++hh) {
+                float x = sr[0][hh];
+#pragma unroll
+                for (int it = 1; it < KIT; ++it) x = j == it ? sr[it][hh] : x;
+                we[hh] = in_j ? expf(x - m[hh]) : 0.0f;
+            }
+            auto add_step = [&](auto step) __attribute__((always_inline)) {
+                constexpr int it = decltype(step)::value;
+                const bool in = !MASKED || t + wave * 4 + pg + kStep * it < p1;
 #pragma unroll
                 for (int hh = 0; hh < G; ++hh) {
-                    const float w = in ? expf(sr[it][hh] - m[hh]) : 0.0f;
+                    const float w = dpp<0x55 * it>(we[hh]);  // quad_perm: lane `it` to all four
                     l[hh] += w;
 #pragma unroll
                     for (int e = 0; e < 8; ++e) acc[hh][e] = in ? fmaf(w, v8[it][e], acc[hh][e]) : acc[hh][e];
                 }
+            };
+            add_step(std::integral_constant<int, 0>{});
+            add_step(std::integral_constant<int, 1>{});
+            if constexpr (KIT == 4) {
+                add_step(std::integral_constant<int, 2>{});
+                add_step(std::integral_constant<int, 3>{});
             }
         };
         for (int t = p0; t < p1; t += kTile) {
@@ -1376,13 +1397,10 @@ __global__ __launch_bounds__(WAVES * kWave) void prefill_attn_kernel(const float
     }
 }
 
-// *pos = the chunk's first position (the combine reads it there), *key = 0,
-// *last_pos = the last column's.
-__global__ void prefill_begin_kernel(int* __restrict__ pos, int first, int* __restrict__ last_pos, int last,
-                                     unsigned long long* __restrict__ key) {
+// *pos = the chunk's first position (the combine reads it there), *key = 0.
+__global__ void prefill_begin_kernel(int* __restrict__ pos, int first, unsigned long long* __restrict__ key) {
     if (threadIdx.x == 0) {
         *pos = first;
-        *last_pos = last;
         *key = 0ull;
     }
 }
@@ -1448,13 +1466,14 @@ struct PrefillDeepAttnK {
     static auto fn() { return prefill_attn_kernel<G, Q8, kDeepForm.waves, kDeepForm.tile / (4 * kDeepForm.waves)>; }
 };
 
-// Columns of a chunk: its buffers stay below 250 MB at the largest widths,
-// and from a few hundred columns a longer chunk gains nothing.
-constexpr int kMaxPrefillTokens = 512;
+// Columns of a chunk, and of one launch of its attention (whose partials,
+// 400 KB a column at 24 heads, are the largest buffer).
+constexpr int kMaxPrefillTokens = 1024;
+constexpr int kPrefillAttnCols = 512;
 
 // Work buffer layout of a prefill chunk of up to n tokens (offsets in floats).
 struct PrefillWork {
-    size_t H, QKV, Q, part, O, GU, img, att, h1, gu1, down1, key, last_pos, total;
+    size_t H, QKV, Q, part, O, GU, img, att, h1, gu1, down1, key, total;
     int nsplit;
 };
 
@@ -1473,7 +1492,7 @@ PrefillWork prefill_work(const asdsl_decode_model& m, int n) {
     w.H = take(N * m.hidden);
     w.QKV = take(N * qkv_dim);
     w.Q = take(N * m.n_heads * m.head_dim);
-    w.part = take(N * m.n_heads * w.nsplit * kPartStride);
+    w.part = take((N < kPrefillAttnCols ? N : kPrefillAttnCols) * m.n_heads * w.nsplit * kPartStride);
     w.O = take(N * m.hidden);
     w.GU = take(N * 2 * m.ffn);
     w.img = take((N + kImageCols - 1) / kImageCols * image_bytes(wide) / sizeof(float));
@@ -1483,25 +1502,23 @@ PrefillWork prefill_work(const asdsl_decode_model& m, int n) {
     w.gu1 = take(2 * static_cast<size_t>(m.ffn));
     w.down1 = take(m.hidden);
     w.key = take(2);
-    w.last_pos = take(1);
     w.total = at;
     return w;
 }
 
-// Partials of columns [c_begin, c_end) of a chunk whose column c is at
-// position first + c.
-asdsl_status launch_prefill_attention(const float* Q, const KvCache& kv, bool q8, float* part, int first, int c_begin,
-                                      int c_end, int n_heads, int n_kv, int max_seq, int nsplit, int cus,
+// Partials of n columns, column c at position first + c.
+asdsl_status launch_prefill_attention(const float* Q, const KvCache& kv, bool q8, float* part, int first, int n,
+                                      int n_heads, int n_kv, int max_seq, int nsplit, int cus,
                                       hipStream_t s) {
     // positions of one form and one split size per launch: below 2048 one
     // tile a split, then one tile more from every 2048 positions
-    for (int c0 = c_begin; c0 < c_end;) {
+    for (int c0 = 0; c0 < n;) {
         const int pos = first + c0;
         const bool deep = pos >= kDeepFrom;
         const FoldForm& f = deep ? kDeepForm : kLongForm;
         const int tps = attn_fold_tps(pos, f.tile, f.max_splits);
         const int span = f.tile * f.max_splits;
-        const int c1 = min(c_end, (pos / span + 1) * span - first);
+        const int c1 = min(n, (pos / span + 1) * span - first);
         const int splits = attn_fold_splits(first + c1 - 1, f.tile, f.max_splits);
         // Columns per workgroup: up to 16 share a tile's rows, fewer while
         // that would leave less than two workgroups per compute unit.
@@ -1876,12 +1893,12 @@ extern "C" asdsl_status asdsl_decode_verify(const asdsl_decode_model* model, con
         if (o_form != 0) {
             st = launch("attn_combine_kernel", m.gs_attn == 32 ? attn_combine_kernel<32> : attn_combine_kernel<128>,
                         dim3(m.n_heads, kImageCols), dim3(combine_threads(nsplit)), 0, s, static_cast<const float*>(part), pos,
-                        att, nsplit, m.max_seq, m.max_seq, 0, n, 0, 0, img, fac_of(q_dim), us_of(q_dim));
+                        0, att, nsplit, m.max_seq, m.max_seq, 0, n, 0, 0, img, fac_of(q_dim), us_of(q_dim));
             if (st != ASDSL_OK) return st;
             st = image_gemv(o_form, L.o_meta, L.o_quant, O, m.hidden, q_dim, m.gs_attn);
         } else {
             st = launch("attn_combine_kernel", attn_combine_kernel<0>, dim3(m.n_heads, n), dim3(combine_threads(nsplit)), 0, s,
-                        static_cast<const float*>(part), pos, att, nsplit, m.max_seq, m.max_seq, 0, n, 0, 0,
+                        static_cast<const float*>(part), pos, 0, att, nsplit, m.max_seq, m.max_seq, 0, n, 0, 0,
                         static_cast<uint2*>(nullptr), static_cast<float2*>(nullptr), static_cast<float*>(nullptr));
             if (st != ASDSL_OK) return st;
             st = mfma ? preq2_fused_batch(L.o_meta, L.o_quant, att, O, m.hidden, q_dim, m.gs_attn, n, stream, true,
@@ -1954,7 +1971,6 @@ extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, co
     float* O = base + w.O;
     float* GU = base + w.GU;
     auto* key = reinterpret_cast<unsigned long long*>(base + w.key);
-    int* last_pos = reinterpret_cast<int*>(base + w.last_pos);
     void* image = base + w.img;
     auto* img = reinterpret_cast<uint2*>(base + w.img);
     hipStream_t s = as_hip(stream);
@@ -1980,7 +1996,7 @@ extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, co
     };
 
     asdsl_status st = launch("prefill_begin_kernel", prefill_begin_kernel, dim3(1), dim3(kWave), 0, s, pos, start_pos,
-                             last_pos, start_pos + n - 1, key);
+                             key);
     if (st != ASDSL_OK) return st;
     st = launch("verify_embed_kernel", verify_embed_kernel, dim3((m.hidden + 1023) / 1024, n), dim3(256), 0, s, m.embed,
                 tokens, H, m.hidden, m.vocab, static_cast<unsigned long long*>(nullptr));
@@ -1998,10 +2014,19 @@ extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, co
                     m.n_heads, m.n_kv_heads, m.max_seq, m.rotary_dim / 2);
         if (st != ASDSL_OK) return st;
         if (last && !logits) break;  // the K/V rows are all that the chunk leaves
-        st = launch_prefill_attention(Q, kv, q8, part, start_pos, last ? n - 1 : 0, n, m.n_heads, m.n_kv_heads,
-                                      m.max_seq, w.nsplit, cus, s);
-        if (st != ASDSL_OK) return st;
         const dim3 cthreads(combine_threads(w.nsplit));
+        for (int c0 = last ? n - 1 : 0; c0 < n; c0 += kPrefillAttnCols) {
+            const int nc = n - c0 < kPrefillAttnCols ? n - c0 : kPrefillAttnCols;
+            st = launch_prefill_attention(Q + static_cast<size_t>(c0) * q_dim, kv, q8, part, start_pos + c0, nc,
+                                          m.n_heads, m.n_kv_heads, m.max_seq, w.nsplit, cus, s);
+            if (st != ASDSL_OK) return st;
+            if (last) break;
+            st = launch("attn_combine_kernel", m.gs_attn == 32 ? attn_combine_kernel<32> : attn_combine_kernel<128>,
+                        dim3(m.n_heads, nc), cthreads, 0, s, static_cast<const float*>(part),
+                        static_cast<const int*>(pos), c0, static_cast<float*>(nullptr), w.nsplit, m.max_seq, m.max_seq,
+                        0, n, kLongForm.tile, kLongForm.max_splits, img, fac_of(q_dim), us_of(q_dim));
+            if (st != ASDSL_OK) return st;
+        }
         if (last) {  // only the last token's: the single-token step's launches
             float* att = base + w.att;
             float* h1 = base + w.h1;
@@ -2010,9 +2035,8 @@ extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, co
             const size_t col = static_cast<size_t>(n - 1);
             const float* h = H + col * m.hidden;
             st = launch("attn_combine_kernel", attn_combine_kernel<0>, dim3(m.n_heads), cthreads, 0, s,
-                        static_cast<const float*>(part) + col * m.n_heads * w.nsplit * kPartStride,
-                        static_cast<const int*>(last_pos), att, w.nsplit, m.max_seq, m.max_seq, 0, 1, kLongForm.tile,
-                        kLongForm.max_splits, static_cast<uint2*>(nullptr), static_cast<float2*>(nullptr),
+                        static_cast<const float*>(part), static_cast<const int*>(pos), n - 1, att, w.nsplit, m.max_seq,
+                        m.max_seq, 0, 1, kLongForm.tile, kLongForm.max_splits, static_cast<uint2*>(nullptr), static_cast<float2*>(nullptr),
                         static_cast<float*>(nullptr));
             if (st != ASDSL_OK) return st;
             st = asdsl_gemv_preq2_fused(L.o_meta, L.o_quant, att, O, m.hidden, q_dim, m.gs_attn, stream);
@@ -2034,11 +2058,6 @@ extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, co
             if (st != ASDSL_OK) return st;
             break;
         }
-        st = launch("attn_combine_kernel", m.gs_attn == 32 ? attn_combine_kernel<32> : attn_combine_kernel<128>,
-                    dim3(m.n_heads, n), cthreads, 0, s, static_cast<const float*>(part), static_cast<const int*>(pos),
-                    static_cast<float*>(nullptr), w.nsplit, m.max_seq, m.max_seq, 0, n, kLongForm.tile,
-                    kLongForm.max_splits, img, fac_of(q_dim), us_of(q_dim));
-        if (st != ASDSL_OK) return st;
         st = gemm(L.o_meta, L.o_quant, O, m.hidden, q_dim, m.gs_attn);
         if (st != ASDSL_OK) return st;
         st = norm_then_gemm(O, L.rms_ffn, L.gu_meta, L.gu_quant, GU, 2 * m.ffn, m.gs_ffn);

@@ -29,8 +29,16 @@
 //    activation operands and scales of a step are staged once in LDS for all
 //    of them (two buffers, the next step's loads in flight while the current
 //    one computes; one barrier per step);
+//    Both are laid out in LDS so that no two lanes of a read share a bank
+//    (as first written, 41 % of the cycles of a gate_up launch were bank
+//    conflicts);
 //  - each wave's 16-row weight tile goes through its own LDS area (one 16-byte
 //    load per lane and step, read back as each MFMA's operand dwords).
+// Measured at 517 columns: gate_up 16384x3072 g128 161 us (323 T int8
+// operations a second; 15.4 vector instructions per MFMA, 70 % of the issue
+// slots taken), down 3072x8192 g128 96 us, qkv 5120x3072 g32 70 us, o_proj
+// 3072x3072 g32 44 us; the same columns as 33 launches of the 16-column exact
+// kernel take 380, 280, 290 and 180 us.
 #include <cstdlib>
 
 #include "abi_util.hpp"
@@ -50,10 +58,11 @@ constexpr int kGemmRows = 16 * kGemmWaves;  // rows of a workgroup's tile
 // slice sums of 16 columns).
 constexpr int kOpBytes = 4 * 512;
 __host__ __device__ constexpr int scale_bytes(int gs) { return gs == 32 ? 512 : 128 + 256; }
-// a wave's weight tile of one step: 4 bands x 256 bytes, 64 bytes apart so
-// that the four bands' reads fall on different banks, and its (s, z) pairs
-constexpr int kBandStride = 256 + 64;
-constexpr int kWaveStage = 4 * kBandStride + 256;
+// a wave's weight tile of one step: 4 bands x 256 bytes, spaced so that the
+// 64 lanes of an operand read (4 bands x 4 rows x 4 dwords; rows 16 bytes
+// apart for GS 32, 64 for GS 128) fall on different banks, and its (s, z) pairs
+__host__ __device__ constexpr int band_stride(int gs) { return 256 + (gs == 32 ? 64 : 16); }
+__host__ __device__ constexpr int wave_stage(int gs) { return 4 * band_stride(gs) + 256; }
 
 template <int GS, int CB>
 __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
@@ -65,13 +74,14 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
     constexpr int kStepGroups = GS == 32 ? 4 : 1;  // groups of a step
     constexpr int kClassStride = GS == 32 ? 16 : 4;  // groups between a class's steps
     constexpr int kScale = scale_bytes(GS);
+    constexpr int kBandStride = band_stride(GS);
     constexpr int kBuf = CB * (kOpBytes + kScale);
     constexpr int kOpUnits = CB * kOpBytes / 16;       // 16-byte units of a step's operands
     constexpr int kScaleUnits = CB * kScale / 16;
     constexpr int kOpLoads = (kOpUnits + kGemmThreads - 1) / kGemmThreads;
     static_assert(kScaleUnits <= kGemmThreads, "one scale unit per thread");
     __shared__ __align__(16) uint8_t s_buf[2][kBuf];
-    __shared__ __align__(16) uint8_t s_stage[kGemmWaves][kWaveStage];
+    __shared__ __align__(16) uint8_t s_stage[kGemmWaves][wave_stage(GS)];
 
     // Workgroup -> tile: ids go round the 8 XCDs in turn, so each XCD gets a
     // contiguous run of tiles, column tiles inside row tiles: the row tile's
@@ -112,7 +122,11 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
         const int cb = u / (kOpBytes / 16);
         const int blk = min(ct * CB + cb, nblk - 1);
         op_src[i] = image + static_cast<size_t>(blk) * image_bytes(K) + (u % (kOpBytes / 16)) * 16;
-        op_dst[i] = cb * kOpBytes + (u % (kOpBytes / 16)) * 16;
+        // a unit is chunks 2h and 2h + 1 (h = u & 1) of a column's 32-element
+        // slice; in LDS a slice is [chunk][column] (the image: [column][chunk]),
+        // so that lane (r16, q) reads the 8 bytes at 8 * lane
+        const int e = u % 32;
+        op_dst[i] = cb * kOpBytes + (u % (kOpBytes / 16)) / 32 * 512 + (e & 1) * 256 + (e >> 1) * 8;
     }
     constexpr int kOpStep = UPS * 512;  // image bytes per group
     const uint8_t* sc_src;
@@ -141,7 +155,10 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
     };
     auto store_shared = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < kOpLoads; ++i) *reinterpret_cast<uint4*>(s_buf[b] + op_dst[i]) = ov[i];
+        for (int i = 0; i < kOpLoads; ++i) {
+            *reinterpret_cast<uint2*>(s_buf[b] + op_dst[i]) = make_uint2(ov[i].x, ov[i].y);
+            *reinterpret_cast<uint2*>(s_buf[b] + op_dst[i] + 128) = make_uint2(ov[i].z, ov[i].w);
+        }
         *reinterpret_cast<uint4*>(s_buf[b] + sc_dst) = sv;
     };
     // the wave reads back only what it wrote; its LDS operations complete in order
@@ -224,7 +241,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
 #pragma unroll
                     for (int cb = 0; cb < CB; ++cb) {
                         const uint64_t b =
-                            *reinterpret_cast<const uint64_t*>(ops + cb * kOpBytes + k * 512 + (r16 * 4 + q) * 8);
+                            *reinterpret_cast<const uint64_t*>(ops + cb * kOpBytes + k * 512 + lane * 8);
                         float xs = 0.0f, xu;
                         if constexpr (GS == 32) {
                             const float2 f = *reinterpret_cast<const float2*>(ops + CB * kOpBytes + cb * kScale +

@@ -591,7 +591,7 @@ asdsl_status asdsl_decode_verify(const asdsl_decode_model* model, const int* tok
                                  float* logits, int* next_tokens, void* work, asdsl_stream_t stream);
 
 /* Bytes of device work buffer asdsl_decode_prefill needs for up to max_tokens
- * tokens (1..512); 0 for an invalid model or count. */
+ * tokens (1..1024); 0 for an invalid model or count. */
 size_t asdsl_decode_prefill_work_bytes(const asdsl_decode_model* model, int max_tokens);
 
 /* Queues one chunk of a prompt: tokens[0..n) (device) at positions start_pos
@@ -600,7 +600,7 @@ size_t asdsl_decode_prefill_work_bytes(const asdsl_decode_model* model, int max_
  * the last token's logits and *token = their greedy argmax; *pos = start_pos +
  * n (device ints; *pos is used as scratch meanwhile).  What it writes is what
  * asdsl_decode_token on each token in turn leaves, bit for bit.  1 <= n <=
- * 512, start_pos + n <= max_seq; work: asdsl_decode_prefill_work_bytes(model,
+ * 1024, start_pos + n <= max_seq; work: asdsl_decode_prefill_work_bytes(model,
  * >= n) bytes, 256-byte aligned.  ASDSL_ERR_UNSUPPORTED (nothing queued) under
  * ASDSL_HIP_NORM_FACTORED.  The reference feeds a prompt one forward_token
  * per token (asdsl/kernels/native/unified_engine.cpp:1339-1688). */

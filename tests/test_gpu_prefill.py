@@ -39,12 +39,13 @@ def _compare(cfg, plens, seed=5):
 
 # 4: the smallest chunk; 16 and 17: one column block and the first of two; 64
 # and 65: a workgroup's 4 blocks and a tile of positions, and one past; 512 and
-# 530: a whole chunk, and a second one
+# 530: the columns of an attention launch, and a second one; 1024 and 1030: a
+# whole chunk, and two
 @pytest.mark.parametrize("kv", ["fp16", "int8"])
 def test_prompt_lengths(gpu, kv):
     from asdsl.engine import DecodeConfig
 
-    _compare(DecodeConfig(n_layers=2, vocab=4096, max_seq=576, kv_format=kv), (4, 16, 17, 64, 65, 197, 512, 530))
+    _compare(DecodeConfig(n_layers=2, vocab=4096, max_seq=1088, kv_format=kv), (4, 16, 17, 64, 65, 197, 512, 530, 1024, 1030))
 
 
 # group sizes in both places, query heads per KV head 1, 2 and 4, and in_features
