@@ -171,26 +171,45 @@ def check(status: int, fn: str) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(LIB, name)(*args), name)
+    status = getattr(LIB, name)(*args)
+    if status:
+        check(status, name)
 
 
 # ----------------------------------------------------------------- buffers
-def _torch():
-    import torch  # imported lazily: argument checks must not need it
+_TORCH = None
 
-    return torch
+
+def _torch():
+    global _TORCH
+    if _TORCH is None:
+        import torch  # imported lazily: argument checks must not need it
+
+        _TORCH = torch
+    return _TORCH
+
+
+_DEVICES: dict = {}  # torch.device by index, once a HIP device was found usable
 
 
 def device() -> "torch.device":
     torch = _torch()
-    if not torch.cuda.is_available():
+    if not _DEVICES and not torch.cuda.is_available():
         raise RuntimeError("no usable HIP device (torch.cuda.is_available() is False)")
-    return torch.device("cuda", torch.cuda.current_device())
+    index = torch.cuda.current_device()
+    dev = _DEVICES.get(index)
+    if dev is None:
+        dev = _DEVICES[index] = torch.device("cuda", index)
+    return dev
 
 
 def stream_handle() -> int:
+    """The current stream of the current device."""
     torch = _torch()
-    return int(torch.cuda.current_stream().cuda_stream)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # without a Stream object: 1 us less
+    if raw is None:
+        return int(torch.cuda.current_stream().cuda_stream)
+    return raw(torch.cuda.current_device())
 
 
 _NP_TO_TORCH = {
@@ -231,9 +250,14 @@ def to_device(a, np_dtype) -> "torch.Tensor":
     return torch.from_numpy(arr).to(device(), non_blocking=False)
 
 
+_EMPTY_DTYPE: dict = {}
+
+
 def empty_device(shape, np_dtype) -> "torch.Tensor":
     torch = _torch()
-    tdt = getattr(torch, _NP_TO_TORCH[np.dtype(np_dtype)])
+    tdt = _EMPTY_DTYPE.get(np_dtype)
+    if tdt is None:
+        tdt = _EMPTY_DTYPE[np_dtype] = getattr(torch, _NP_TO_TORCH[np.dtype(np_dtype)])
     return torch.empty(shape, dtype=tdt, device=device())
 
 
