@@ -80,6 +80,7 @@ SIGNATURES: dict[str, list] = {
     "asdsl_sparse_down_proj_T_noalloc": [_P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _P],
     "asdsl_sparse_down_proj_T_ws": [_P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "asdsl_gemv_preq2_fused_batch_work_bytes": [_I],
+    "asdsl_gemv_preq2_fused_batch_work_bytes_n": [_I, _I],
     "asdsl_gemv_preq2_fused_batch_ws": [_P, _P, _P, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "asdsl_affine_batch_work_bytes": [_I, _I, _I],
     "asdsl_gemv_q4_packed_ws": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
@@ -116,6 +117,7 @@ _RESTYPE = {"asdsl_last_error": ctypes.c_char_p, "asdsl_attention_work_floats": 
             "asdsl_decode_flags_offset": ctypes.c_size_t,
             "asdsl_sparse_down_work_bytes": ctypes.c_size_t, "asdsl_grid_sync_probe_work_bytes": ctypes.c_size_t,
             "asdsl_gemv_preq2_fused_batch_work_bytes": ctypes.c_size_t,
+            "asdsl_gemv_preq2_fused_batch_work_bytes_n": ctypes.c_size_t,
             "asdsl_affine_batch_work_bytes": ctypes.c_size_t}
 
 

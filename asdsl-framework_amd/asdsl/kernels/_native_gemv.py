@@ -191,7 +191,7 @@ def gemv_preq2_fused_avx2(meta, quant, x_fp32, y, out_features: int, in_features
     px = c.input(x_fp32, np.float32, n_cols * in_features, "x_fp32")
     py = c.output(y, np.float32, n_cols * out_features, "y")
     if len(xs) == 2:
-        nbytes = int(_hip.LIB.asdsl_gemv_preq2_fused_batch_work_bytes(in_features))
+        nbytes = int(_hip.LIB.asdsl_gemv_preq2_fused_batch_work_bytes_n(in_features, min(max(n_cols, 1), 64)))
         c.run("asdsl_gemv_preq2_fused_batch_ws", pm, pq, px, py, out_features, in_features, group_size, n_cols,
               c.scratch(nbytes, np.uint8), nbytes)
     else:

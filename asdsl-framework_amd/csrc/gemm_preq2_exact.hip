@@ -1,5 +1,5 @@
-// preq2 GEMM of a prompt chunk: Y[n][:] = preq2(W) x_n for any number of
-// activation columns, each column bit for bit what the single-column GEMV
+// preq2 GEMM of a prompt chunk and of batches of more than 16 columns: Y[n][:]
+// = preq2(W) x_n for any number of activation columns, each column bit for bit what the single-column GEMV
 // gives on it (plan_preq2's K split and lane layout), so that a prompt run in
 // chunks leaves the K/V rows and logits of one step per token.  The reference
 // feeds a prompt one forward_token per token
@@ -64,7 +64,14 @@ __host__ __device__ constexpr int scale_bytes(int gs) { return gs == 32 ? 512 : 
 __host__ __device__ constexpr int band_stride(int gs) { return 256 + (gs == 32 ? 64 : 16); }
 __host__ __device__ constexpr int wave_stage(int gs) { return 4 * band_stride(gs) + 256; }
 
-template <int GS, int CB>
+// SPLIT: the workgroup's waves take one class each of the same 16 rows, with
+// operands, scales and weights all in the wave's own LDS area and no barrier
+// but the one per K range that adds the classes.  A quarter of the steps per
+// wave and four times the workgroups, for column counts that leave the other
+// form with about one wave per SIMD: its time is then the steps' memory
+// latency, 0.6 to 0.8 us each (down 3072x8192 g128 at 24 columns: 13.2 us split,
+// 37.8 not).
+template <int GS, int CB, bool SPLIT>
 __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
     const uint32_t* __restrict__ meta, const uint8_t* __restrict__ quant, const uint8_t* __restrict__ image,
     float* __restrict__ Y, int M, int K, int ncols, int KS, int NU, int nrt, int nct, int per_xcd) {
@@ -78,10 +85,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
     constexpr int kBuf = CB * (kOpBytes + kScale);
     constexpr int kOpUnits = CB * kOpBytes / 16;       // 16-byte units of a step's operands
     constexpr int kScaleUnits = CB * kScale / 16;
-    constexpr int kOpLoads = (kOpUnits + kGemmThreads - 1) / kGemmThreads;
-    static_assert(kScaleUnits <= kGemmThreads, "one scale unit per thread");
-    __shared__ __align__(16) uint8_t s_buf[2][kBuf];
+    constexpr int kLoaders = SPLIT ? kWave : kGemmThreads;  // threads that stage one operand buffer
+    constexpr int kOpLoads = (kOpUnits + kLoaders - 1) / kLoaders;
+    static_assert(kScaleUnits <= kLoaders, "one scale unit per thread");
+    __shared__ __align__(16) uint8_t s_bufs[SPLIT ? kGemmWaves : 2][kBuf];
     __shared__ __align__(16) uint8_t s_stage[kGemmWaves][wave_stage(GS)];
+    __shared__ float s_red[SPLIT ? 2 : 1][SPLIT ? kGemmWaves : 1][SPLIT ? CB * 4 : 1][kWave];
 
     // Workgroup -> tile: ids go round the 8 XCDs in turn, so each XCD gets a
     // contiguous run of tiles, column tiles inside row tiles: the row tile's
@@ -100,8 +109,10 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
     const int q = lane >> 4;
     const int nbands = (M + 3) >> 2;
     const int nblk = (ncols + kImageCols - 1) / kImageCols;
-    const int row0 = rt * kGemmRows + wave * 16;
+    const int row0 = SPLIT ? rt * 16 : rt * kGemmRows + wave * 16;
     uint8_t* stage = s_stage[wave];
+    uint8_t (*s_buf)[kBuf] = SPLIT ? s_bufs + wave : s_bufs;
+    const int loader = SPLIT ? lane : tid;
 
     // rows past M read the last band / row and are never stored
     const uint8_t* wband = quant + static_cast<size_t>(min((row0 >> 2) + (lane >> 4), nbands - 1)) * G * kGroupBytes +
@@ -118,7 +129,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
     int op_dst[kOpLoads];
 #pragma unroll
     for (int i = 0; i < kOpLoads; ++i) {
-        const int u = min(i * kGemmThreads + tid, kOpUnits - 1);
+        const int u = min(i * kLoaders + loader, kOpUnits - 1);
         const int cb = u / (kOpBytes / 16);
         const int blk = min(ct * CB + cb, nblk - 1);
         op_src[i] = image + static_cast<size_t>(blk) * image_bytes(K) + (u % (kOpBytes / 16)) * 16;
@@ -132,7 +143,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
     const uint8_t* sc_src;
     int sc_dst, sc_step;
     {
-        const int u = min(tid, kScaleUnits - 1);
+        const int u = min(loader, kScaleUnits - 1);
         const int cb = u / (kScale / 16);
         const int e = u % (kScale / 16);
         const int blk = min(ct * CB + cb, nblk - 1);
@@ -178,12 +189,15 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
 #pragma unroll
         for (int v = 0; v < 4; ++v) tA[cb][v] = tB[cb][v] = sum[cb][v] = 0.0f;
 
-    load_step(0);
+    const int w_begin = SPLIT ? wave : 0;
+    const int w_end = SPLIT ? wave + 1 : 4;
+    const int first = group_of(0, w_begin, 0);
+    load_step(first < G ? first : 0);
     store_shared(0);
     int buf = 0;
     const v4i32 zero = {0, 0, 0, 0};
     for (int ks = 0; ks < KS; ++ks) {
-        for (int w = 0; w < 4; ++w) {
+        for (int w = w_begin; w < w_end; ++w) {
             float acc[CB][4][4];  // [column block][row 4q + v][accumulator j]
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb)
@@ -195,10 +209,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
                 const int g = group_of(ks, w, st);
                 if (g >= G) break;
                 store_wave();
-                __syncthreads();  // buffer `buf` is complete; the other one is free
+                if constexpr (SPLIT) __builtin_amdgcn_wave_barrier();
+                else __syncthreads();  // buffer `buf` is complete; the other one is free
                 // the next step's loads (after the last step: this one's again)
                 int gn = group_of(ks, w, st + 1);
-                if (st + 1 == NU || gn >= G) gn = w < 3 ? group_of(ks, w + 1, 0) : group_of(ks + 1, 0, 0);
+                if (st + 1 == NU || gn >= G)
+                    gn = w + 1 < w_end ? group_of(ks, w + 1, 0) : group_of(ks + 1, w_begin, 0);
                 load_step(gn < G ? gn : g);
                 __builtin_amdgcn_sched_barrier(0);
 
@@ -263,7 +279,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                buf ^= 1;
+                if constexpr (!SPLIT) buf ^= 1;
                 store_shared(buf);
             }
             // the class's in-row fold, then the classes and the K ranges
@@ -281,7 +297,20 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
 #pragma unroll
                     for (int v = 0; v < 4; ++v) f(tA[cb][v], tB[cb][v], sum[cb][v], r[cb][v]);
             };
-            if (w == 0) {
+            if constexpr (SPLIT) {  // wave v adds the classes' value v of every block
+                float (*red)[CB * 4][kWave] = s_red[ks & 1];
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) red[wave][cb * 4 + v][lane] = r[cb][v];
+                __syncthreads();  // every wave passes it once per K range
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+                    const int i = cb * 4 + wave;
+                    const float p = (red[0][i][lane] + red[1][i][lane]) + (red[2][i][lane] + red[3][i][lane]);
+                    sum[cb][0] = ks == 0 ? p : sum[cb][0] + p;
+                }
+            } else if (w == 0) {
                 each([](float& a, float&, float&, float x) { a = x; });
             } else if (w == 1) {
                 each([](float& a, float&, float&, float x) { a = a + x; });
@@ -294,24 +323,33 @@ __global__ __launch_bounds__(kGemmThreads, 2) void preq2_gemm_exact_kernel(
             }
         }
     }
-    const int row = row0 + 4 * q;
+    const int row = row0 + 4 * q + (SPLIT ? wave : 0);
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
         const int n = (ct * CB + cb) * kImageCols + r16;
-        if (n < ncols && row < M)  // M % 4 == 0
-            *reinterpret_cast<float4*>(Y + static_cast<size_t>(n) * M + row) =
-                make_float4(sum[cb][0], sum[cb][1], sum[cb][2], sum[cb][3]);
+        if (n >= ncols) continue;
+        float* y = Y + static_cast<size_t>(n) * M + row;
+        if constexpr (SPLIT) {
+            if (row < M) *y = sum[cb][0];
+        } else if ((M & 3) == 0) {
+            if (row < M) *reinterpret_cast<float4*>(y) = make_float4(sum[cb][0], sum[cb][1], sum[cb][2], sum[cb][3]);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (row + v < M) y[v] = sum[cb][v];
+        }
     }
 }
 
-template <int GS, int CB>
+template <int GS, int CB, bool SPLIT = false>
 asdsl_status launch_gemm(const uint8_t* meta, const uint8_t* quant, const void* image, float* Y, int M, int K,
                          int ncols, int ks, int nu, hipStream_t s) {
-    const int nrt = (M + kGemmRows - 1) / kGemmRows;
+    const int rows = SPLIT ? 16 : kGemmRows;
+    const int nrt = (M + rows - 1) / rows;
     const int nblk = (ncols + kImageCols - 1) / kImageCols;
     const int nct = (nblk + CB - 1) / CB;
     const int per_xcd = (nrt * nct + 7) / 8;
-    return launch("preq2_gemm_exact_kernel", preq2_gemm_exact_kernel<GS, CB>, dim3(8 * per_xcd), dim3(kGemmThreads), 0,
+    return launch("preq2_gemm_exact_kernel", preq2_gemm_exact_kernel<GS, CB, SPLIT>, dim3(8 * per_xcd), dim3(kGemmThreads), 0,
                   s, reinterpret_cast<const uint32_t*>(meta), quant, static_cast<const uint8_t*>(image), Y, M, K,
                   ncols, ks, nu, nrt, nct, per_xcd);
 }
@@ -326,7 +364,7 @@ asdsl_status asdsl::preq2_gemm_exact(const uint8_t* meta, const uint8_t* quant, 
                                      asdsl_stream_t stream) {
     const int M = out_features, K = in_features;
     ASDSL_CHECK_ARG(meta && quant && image && Y, "gemm_preq2_exact: null pointer");
-    ASDSL_CHECK_ARG((group_size == 32 || group_size == 128) && M > 0 && M % 4 == 0 && K > 0 && K % 128 == 0 &&
+    ASDSL_CHECK_ARG((group_size == 32 || group_size == 128) && M > 0 && K > 0 && K % 128 == 0 &&
                         K / 32 <= 640 && n_cols > 0,
                     "gemm_preq2_exact: invalid dimensions");
     ASDSL_CHECK_ARG(reinterpret_cast<uintptr_t>(image) % 16 == 0 && reinterpret_cast<uintptr_t>(quant) % 16 == 0 &&
@@ -337,25 +375,43 @@ asdsl_status asdsl::preq2_gemm_exact(const uint8_t* meta, const uint8_t* quant, 
     bool exact = false;
     preq2_plan_shape(M, K, cus, &lks, &nu, &waves, &exact);
     const int ks = 1 << lks;
-    // Column blocks per workgroup: a block more shares the unpacked weights
-    // and (s, z) pairs among more MFMAs (about 60 vector instructions per
-    // step of 4 MFMAs per block, each 16) but leaves fewer workgroups; taken
-    // is the smallest product of rounds over the compute units and cost.
+    hipStream_t s = as_hip(stream);
     const int nrt = (M + kGemmRows - 1) / kGemmRows;
     const int nblk = (n_cols + kImageCols - 1) / kImageCols;
+    // Up to 4.5 tiles of 64 rows x 16 columns per compute unit the split form
+    // (us, split against not: o_proj 3072x3072 g32 at 80 columns, 0.9 tiles,
+    // 13.2 / 18.3; down 3072x8192 g128 at 256, 3 tiles, 46.0 / 76.0; gate_up
+    // 16384x3072 g128 at 64, 4 tiles, 27.6 / 33.0, at 80, 5 tiles, 36.8 /
+    // 32.2; qkv 5120x3072 g32 at 256, 5 tiles, 35.7 / 36.5), with one block a
+    // workgroup while four workgroups per compute unit hold them all (down at
+    // 80 columns, 960 workgroups: 20.1 / 24.2 with two; at 128, 1536: 32.4 /
+    // 24.6).
+    if (2LL * nrt * nblk <= 9LL * cus) {
+        const bool one = nblk == 1 || static_cast<long long>((M + 15) / 16) * nblk <= 4LL * cus;
+        if (group_size == 32)
+            return one ? launch_gemm<32, 1, true>(meta, quant, image, Y, M, K, n_cols, ks, nu, s)
+                       : launch_gemm<32, 2, true>(meta, quant, image, Y, M, K, n_cols, ks, nu, s);
+        return one ? launch_gemm<128, 1, true>(meta, quant, image, Y, M, K, n_cols, ks, nu, s)
+                   : launch_gemm<128, 2, true>(meta, quant, image, Y, M, K, n_cols, ks, nu, s);
+    }
+    // Column blocks per workgroup otherwise: a block more shares the unpacked
+    // weights and (s, z) pairs among more MFMAs (about 60 vector instructions
+    // per step of 4 MFMAs per block, each 16) but leaves fewer workgroups;
+    // taken is the smallest product of rounds over the compute units and cost.
     auto cost = [&](int cb) {
         const long long wgs = static_cast<long long>(nrt) * ((nblk + cb - 1) / cb);
         return ((wgs + cus - 1) / cus) * (60 + 64 * cb);
     };
     int cb = 4;
-    if (cost(2) < cost(cb)) cb = 2;
-    if (cost(1) < cost(cb)) cb = 1;
-    hipStream_t s = as_hip(stream);
+    for (int c = 3; c >= 1; --c)
+        if (cost(c) < cost(cb)) cb = c;
     if (group_size == 32)
         return cb == 4   ? launch_gemm<32, 4>(meta, quant, image, Y, M, K, n_cols, ks, nu, s)
+               : cb == 3 ? launch_gemm<32, 3>(meta, quant, image, Y, M, K, n_cols, ks, nu, s)
                : cb == 2 ? launch_gemm<32, 2>(meta, quant, image, Y, M, K, n_cols, ks, nu, s)
                          : launch_gemm<32, 1>(meta, quant, image, Y, M, K, n_cols, ks, nu, s);
     return cb == 4   ? launch_gemm<128, 4>(meta, quant, image, Y, M, K, n_cols, ks, nu, s)
+           : cb == 3 ? launch_gemm<128, 3>(meta, quant, image, Y, M, K, n_cols, ks, nu, s)
            : cb == 2 ? launch_gemm<128, 2>(meta, quant, image, Y, M, K, n_cols, ks, nu, s)
                      : launch_gemm<128, 1>(meta, quant, image, Y, M, K, n_cols, ks, nu, s);
 }

@@ -197,8 +197,13 @@ static_assert(kMfmaCols == kImageCols, "one image layout");
 
 template <int GS>
 __global__ __launch_bounds__(256) void batch_quantize_kernel(const float* __restrict__ X, uint2* __restrict__ img,
-                                                             float2* __restrict__ fac, int K, int ncols) {
-    const int n = static_cast<int>(blockIdx.y);
+                                                             float2* __restrict__ fac, float* __restrict__ us, int K,
+                                                             int ncols) {
+    const int n = static_cast<int>(blockIdx.y);  // its image is n / kImageCols
+    const size_t at = image_at(n, K);
+    img += at / sizeof(uint2);
+    fac += at / sizeof(float2);
+    if (us) us += at / sizeof(float);
     const int c = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
     const int nchunk = K >> 3;  // a multiple of 4: lanes past the end form whole groups
     const int cc = min(c, nchunk - 1);
@@ -212,7 +217,7 @@ __global__ __launch_bounds__(256) void batch_quantize_kernel(const float* __rest
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = 0.0f;
     }
-    image_store8<GS>(v, c, n, c < nchunk, img, fac);
+    image_store8<GS>(v, c, n % kImageCols, c < nchunk, img, fac, us);
 }
 
 typedef int v4i32 __attribute__((ext_vector_type(4)));
@@ -222,18 +227,24 @@ typedef int v4i32 __attribute__((ext_vector_type(4)));
 // bands of a tile fall on different LDS banks.
 __host__ __device__ constexpr int mfma_band_bytes(int gs, int gpw) { return gpw * (gs * 2) + 64; }
 // Per wave: the weight staging area (4 bands of one tile) and the wave's
-// (xs, X*xs) pairs (GPW groups x 16 columns x 8 B); per workgroup: two
-// buffers of the fixed-order K-slice sum.
-__host__ __device__ constexpr int mfma_wave_bytes(int gs, int gpw) { return 4 * mfma_band_bytes(gs, gpw) + gpw * 128; }
-__host__ __device__ constexpr size_t mfma_lds_bytes(int gs, int gpw, int waves) {
-    return static_cast<size_t>(waves) * mfma_wave_bytes(gs, gpw) + 2 * static_cast<size_t>(waves) * 4 * kWave * 4;
+// (xs, X*xs) pairs (GPW groups x 16 columns x 8 B per column block); per
+// workgroup: two buffers of the fixed-order K-slice sum.
+__host__ __device__ constexpr int mfma_wave_bytes(int gs, int gpw, int cb) {
+    return 4 * mfma_band_bytes(gs, gpw) + cb * gpw * 128;
+}
+__host__ __device__ constexpr size_t mfma_lds_bytes(int gs, int gpw, int waves, int cb) {
+    return static_cast<size_t>(waves) * mfma_wave_bytes(gs, gpw, cb) + 2 * static_cast<size_t>(waves) * cb * 4 * kWave * 4;
 }
 
 // Workgroups loop over 16-row tiles (tile = blockIdx.x, += gridDim.x).  With
 // PF each wave requests the next tile's weights and (s, z) pairs before it
 // computes the current one, so HBM streams while the fp32 epilogue runs;
 // without PF (one tile per workgroup) the second register set is not needed.
-template <int GS, int GPW, int W, bool PF>
+// CB blocks of 16 columns (images image_bytes(K) apart) share a pass over the
+// weights: what bounds the kernel past 16 columns is the fp32 epilogue, 16
+// vector instructions per MFMA, and the weights' unpacking and decoding, about
+// 10 more per slice, are then done once for all blocks.
+template <int GS, int GPW, int W, bool PF, int CB>
 __global__ __launch_bounds__(W * kWave) void preq2_batch_mfma_kernel(const uint32_t* __restrict__ meta,
                                                                     const uint8_t* __restrict__ quant,
                                                                     const uint2* __restrict__ img,
@@ -255,9 +266,10 @@ __global__ __launch_bounds__(W * kWave) void preq2_batch_mfma_kernel(const uint3
     const int g0 = wave * GPW;
     const int ntiles = (M + 15) >> 4;
     const int nbands = (M + 3) >> 2;
-    uint8_t* stage = lds + static_cast<size_t>(wave) * mfma_wave_bytes(GS, GPW);
-    uint8_t* wfac = stage + 4 * kBand;
-    float* red = reinterpret_cast<float*>(lds + static_cast<size_t>(W) * mfma_wave_bytes(GS, GPW));  // [2][W][4][kWave]
+    uint8_t* stage = lds + static_cast<size_t>(wave) * mfma_wave_bytes(GS, GPW, CB);
+    uint8_t* wfac = stage + 4 * kBand;  // [CB][GPW][16] pairs
+    // [2][W][4 * CB][kWave]
+    float* red = reinterpret_cast<float*>(lds + static_cast<size_t>(W) * mfma_wave_bytes(GS, GPW, CB));
 
     // Weights: a tile's four bands x GPW groups are contiguous runs of
     // GPW*GS*2 bytes in HBM (within a group, 16-byte unit r*UPS + t holds
@@ -298,23 +310,30 @@ __global__ __launch_bounds__(W * kWave) void preq2_batch_mfma_kernel(const uint3
 
     // activation operands (column r16, chunk q of each slice of the wave's
     // groups) and the wave's (xs, X*xs) pairs (GPW*128 contiguous bytes, to LDS)
-    long a[GPW][UPS];
-#pragma unroll
-    for (int j = 0; j < GPW; ++j)
-#pragma unroll
-        for (int t = 0; t < UPS; ++t) {
-            const uint2 v = img[(static_cast<size_t>((g0 + j) * UPS + t) * kMfmaCols + r16) * 4 + q];
-            a[j][t] = static_cast<long>(static_cast<uint64_t>(v.x) | (static_cast<uint64_t>(v.y) << 32));
-        }
+    long a[CB][GPW][UPS];
     constexpr int kFacLoads = (GPW * 8 + kWave - 1) / kWave;
-    uint4 fv[kFacLoads];
-    const uint4* fsrc = reinterpret_cast<const uint4*>(fac + static_cast<size_t>(g0) * kMfmaCols);
+    uint4 fv[CB][kFacLoads];
 #pragma unroll
-    for (int i = 0; i < kFacLoads; ++i) fv[i] = fsrc[min(i * kWave + lane, GPW * 8 - 1)];
+    for (int cb = 0; cb < CB; ++cb) {
+        const size_t at = static_cast<size_t>(cb) * image_bytes(K);
+#pragma unroll
+        for (int j = 0; j < GPW; ++j)
+#pragma unroll
+            for (int t = 0; t < UPS; ++t) {
+                const uint2 v = img[at / sizeof(uint2) + (static_cast<size_t>((g0 + j) * UPS + t) * kMfmaCols + r16) * 4 + q];
+                a[cb][j][t] = static_cast<long>(static_cast<uint64_t>(v.x) | (static_cast<uint64_t>(v.y) << 32));
+            }
+        const uint4* fsrc = reinterpret_cast<const uint4*>(fac + at / sizeof(float2) + static_cast<size_t>(g0) * kMfmaCols);
+#pragma unroll
+        for (int i = 0; i < kFacLoads; ++i) fv[cb][i] = fsrc[min(i * kWave + lane, GPW * 8 - 1)];
+    }
     load_tile(w0, m0, tile);  // the grid never exceeds the tile count
 #pragma unroll
-    for (int i = 0; i < kFacLoads; ++i)
-        if (i * kWave + lane < GPW * 8) reinterpret_cast<uint4*>(wfac)[i * kWave + lane] = fv[i];
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int i = 0; i < kFacLoads; ++i)
+            if (i * kWave + lane < GPW * 8)
+                reinterpret_cast<uint4*>(wfac + cb * (GPW * 128))[i * kWave + lane] = fv[cb][i];
 
     const v4i32 zero = {0, 0, 0, 0};
     const int rd = (r16 >> 2) * kBand + (r16 & 3) * (UPS * 16) + q * 4;  // row r16, chunk q of slice 0
@@ -341,41 +360,54 @@ __global__ __launch_bounds__(W * kWave) void preq2_batch_mfma_kernel(const uint3
         if constexpr (decltype(prefetch)::value) load_tile(wn, mn, tile + step);
         __builtin_amdgcn_sched_barrier(0);
 
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        float acc[CB][4];
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[cb][v] = 0.0f;
 #pragma unroll
         for (int j = 0; j < GPW; ++j) {
-            const float4 f0 = reinterpret_cast<const float4*>(wfac + j * 128 + q * 32)[0];
-            const float4 f1 = reinterpret_cast<const float4*>(wfac + j * 128 + q * 32)[1];
-            const float xs[4] = {f0.x, f0.z, f1.x, f1.z};
-            const float xx[4] = {f0.y, f0.w, f1.y, f1.w};
-            v4i32 d = zero;
+            v4i32 d[CB];
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) d[cb] = zero;
 #pragma unroll
             for (int t = 0; t < UPS; ++t) {
                 const uint32_t w = *reinterpret_cast<const uint32_t*>(stage + rd + j * kGroupBytes + t * 16);
                 const uint64_t b = static_cast<uint64_t>(w & 0x0F0F0F0Fu) |
                                    (static_cast<uint64_t>((w >> 4) & 0x0F0F0F0Fu) << 32);
-                d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[j][t], static_cast<long>(b), d, 0, 0, 0);
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+                    d[cb] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[cb][j][t], static_cast<long>(b), d[cb], 0, 0, 0);
             }
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                acc[v] = fmaf(static_cast<float>(d[v]), sf[j] * xs[v], acc[v]);
-                acc[v] = fmaf(zsf[j], xx[v], acc[v]);
+            for (int cb = 0; cb < CB; ++cb) {
+                const float4* f = reinterpret_cast<const float4*>(wfac + (cb * GPW + j) * 128 + q * 32);
+                const float4 f0 = f[0], f1 = f[1];
+                const float xs[4] = {f0.x, f0.z, f1.x, f1.z};
+                const float xx[4] = {f0.y, f0.w, f1.y, f1.w};
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    acc[cb][v] = fmaf(static_cast<float>(d[cb][v]), sf[j] * xs[v], acc[cb][v]);
+                    acc[cb][v] = fmaf(zsf[j], xx[v], acc[cb][v]);
+                }
             }
         }
 
         // add the W K-slices in fixed order; the two buffers alternate, so
         // one barrier per tile suffices
-        float* rb = red + parity * (W * 4 * kWave);
+        float* rb = red + parity * (W * CB * 4 * kWave);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) rb[(wave * 4 + v) * kWave + lane] = acc[v];
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) rb[((wave * CB + cb) * 4 + v) * kWave + lane] = acc[cb][v];
         __syncthreads();
-        for (int e = static_cast<int>(threadIdx.x); e < 4 * kWave; e += W * kWave) {
+        for (int e = static_cast<int>(threadIdx.x); e < CB * 4 * kWave; e += W * kWave) {
             float sum = rb[e];
 #pragma unroll
-            for (int k = 1; k < W; ++k) sum += rb[k * 4 * kWave + e];
-            const int v = e / kWave;
+            for (int k = 1; k < W; ++k) sum += rb[k * CB * 4 * kWave + e];
+            const int v = e / kWave;  // 4 * block + register
             const int l = e & (kWave - 1);
-            const int n = 4 * (l >> 4) + v;
+            const int n = kMfmaCols * (v >> 2) + 4 * (l >> 4) + (v & 3);
             const int row = tile * 16 + (l & 15);
             if (n < ncols && row < M) Y[static_cast<size_t>(n) * M + row] = sum;
         }
@@ -448,18 +480,57 @@ asdsl_status launch_mfma_shape(const MfmaPlan& p, const uint32_t* m, const uint8
                                const float2* fac, float* Y, int M, int K, int ncols, hipStream_t s) {
     if constexpr (W < 16) {  // 16 waves: 128 registers, no room for the second register set
         if (p.prefetch)
-            return launch("preq2_batch_mfma_kernel", preq2_batch_mfma_kernel<GS, GPW, W, true>, dim3(p.grid),
-                          dim3(W * kWave), mfma_lds_bytes(GS, GPW, W), s, m, q, img, fac, Y, M, K, ncols);
+            return launch("preq2_batch_mfma_kernel", preq2_batch_mfma_kernel<GS, GPW, W, true, 1>, dim3(p.grid),
+                          dim3(W * kWave), mfma_lds_bytes(GS, GPW, W, 1), s, m, q, img, fac, Y, M, K, ncols);
     }
-    return launch("preq2_batch_mfma_kernel", preq2_batch_mfma_kernel<GS, GPW, W, false>, dim3(p.grid),
-                  dim3(W * kWave), mfma_lds_bytes(GS, GPW, W), s, m, q, img, fac, Y, M, K, ncols);
+    return launch("preq2_batch_mfma_kernel", preq2_batch_mfma_kernel<GS, GPW, W, false, 1>, dim3(p.grid),
+                  dim3(W * kWave), mfma_lds_bytes(GS, GPW, W, 1), s, m, q, img, fac, Y, M, K, ncols);
+}
+
+// 17 to 64 columns at W <= 8 waves: as many column blocks a launch as the
+// operand registers (2 per slice of a wave's K share and block) leave room
+// for without spilling, the blocks spread evenly over the launches.
+template <int GS, int GPW, int W>
+asdsl_status launch_mfma_blocks(const MfmaPlan& p, const uint32_t* m, const uint8_t* q, const uint2* img,
+                                const float2* fac, float* Y, int M, int K, int ncols, hipStream_t s) {
+    constexpr int kSlices = GPW * (GS / 32);
+    constexpr int kMaxCb = 48 / kSlices < 4 ? 48 / kSlices : 4;  // 4 to 12 slices, 3 at 16, 2 at 20
+    const int blocks = (ncols + kMfmaCols - 1) / kMfmaCols;
+    const int launches = (blocks + kMaxCb - 1) / kMaxCb;
+    const int per = (blocks + launches - 1) / launches;
+    for (int b0 = 0; b0 < blocks; b0 += per) {
+        const int cb = blocks - b0 < per ? blocks - b0 : per;
+        const int n0 = b0 * kMfmaCols;
+        const int nc = ncols - n0 < cb * kMfmaCols ? ncols - n0 : cb * kMfmaCols;
+        auto go = [&](auto kern) {
+            return launch("preq2_batch_mfma_kernel", kern, dim3(p.grid), dim3(W * kWave), mfma_lds_bytes(GS, GPW, W, cb),
+                          s, m, q, img + b0 * (image_bytes(K) / sizeof(uint2)),
+                          fac + b0 * (image_bytes(K) / sizeof(float2)), Y + static_cast<size_t>(n0) * M, M, K, nc);
+        };
+        asdsl_status st = ASDSL_ERR_UNSUPPORTED;
+        if (cb == 1) st = go(preq2_batch_mfma_kernel<GS, GPW, W, true, 1>);
+        if (cb == 2) st = go(preq2_batch_mfma_kernel<GS, GPW, W, true, 2>);
+        if constexpr (kMaxCb >= 3) {
+            if (cb == 3) st = go(preq2_batch_mfma_kernel<GS, GPW, W, true, 3>);
+        }
+        if constexpr (kMaxCb >= 4) {
+            if (cb == 4) st = go(preq2_batch_mfma_kernel<GS, GPW, W, true, 4>);
+        }
+        if (st != ASDSL_OK) return st;
+    }
+    return ASDSL_OK;
 }
 
 asdsl_status launch_mfma(const MfmaPlan& p, int gs, const uint32_t* m, const uint8_t* q, const uint2* img,
                          const float2* fac, float* Y, int M, int K, int ncols, hipStream_t s) {
-#define ASDSL_MFMA_CASE(GS_, W_, GPW_)          \
-    if (gs == GS_ && p.waves == W_ && p.gpw == GPW_) \
-        return launch_mfma_shape<GS_, GPW_, W_>(p, m, q, img, fac, Y, M, K, ncols, s);
+#define ASDSL_MFMA_CASE(GS_, W_, GPW_)                                                        \
+    if (gs == GS_ && p.waves == W_ && p.gpw == GPW_) {                                        \
+        if constexpr (W_ <= 8) {                                                              \
+            if (ncols > kMfmaCols)                                                            \
+                return launch_mfma_blocks<GS_, GPW_, W_>(p, m, q, img, fac, Y, M, K, ncols, s); \
+        }                                                                                     \
+        return launch_mfma_shape<GS_, GPW_, W_>(p, m, q, img, fac, Y, M, K, ncols, s);        \
+    }
     ASDSL_MFMA_CASE(32, 8, 12)
     ASDSL_MFMA_CASE(32, 16, 16)
     ASDSL_MFMA_CASE(32, 8, 16)
@@ -1069,8 +1140,42 @@ asdsl_status asdsl::preq2_fused_batch(const uint8_t* meta, const uint8_t* quant,
     static const int mfma_knob = env_knob("ASDSL_HIP_BATCH_MFMA_MIN_N");
     const int mfma_min = mfma_knob > 0 ? mfma_knob : kBatchMfmaMinN;
     const MfmaPlan mp = plan_mfma(M, K, group_size, cus);
-    if (allow_mfma && n_cols >= mfma_min && mp.ok && reinterpret_cast<uintptr_t>(meta) % 16 == 0 &&
-        reinterpret_cast<uintptr_t>(quant) % 4 == 0) {
+    const bool mfma_ok = mp.ok && reinterpret_cast<uintptr_t>(meta) % 16 == 0 &&
+                         reinterpret_cast<uintptr_t>(quant) % 4 == 0;
+    // With the caller's room for an image per 16 columns (the library's own
+    // work buffer holds one), one quantize launch and one pass over the weights:
+    //  - more than 16 columns where the MFMA kernel has a tiling of up to 8
+    //    waves: all column blocks in it, the same bits as 16 columns a launch
+    //    (gate_up 16384x3072 at 45 columns: g32 34.3 -> 21.6 us, g128 27.7 ->
+    //    14.3).  16-wave tilings (in_features 8192) have no registers for a
+    //    second block and stay at 16 columns a launch;
+    //  - no MFMA tiling for in_features: the exact GEMM, the single-column
+    //    GEMV's bits, where that would otherwise run once per column (3.3 us
+    //    each: from 4 columns; 1000x2688 g32 at 4 / 45 columns: 13.4 / 148 ->
+    //    7.8 / 8.3 us) or as dot4 launches of 8 columns (beyond 8; 16384x1536
+    //    g32 at 8 / 16 / 45: dot4 11.3 / 22.1 / 62, the GEMM 10.9 / 11.0 / 19.6).
+    const int images = (n_cols + kMfmaCols - 1) / kMfmaCols;
+    if (allow_mfma && work && work_bytes >= images * image_bytes(K) && reinterpret_cast<uintptr_t>(work) % 256 == 0) {
+        const bool blocks = mfma_ok && mp.waves <= 8 && n_cols > kMfmaCols && n_cols >= mfma_min;
+        const bool per_column = !p.exact || K > 8192;
+        const bool gemm = !mp.ok && K % 128 == 0 && n_cols >= (per_column ? 4 : 9) &&
+                          reinterpret_cast<uintptr_t>(quant) % 16 == 0 && reinterpret_cast<uintptr_t>(meta) % 4 == 0 &&
+                          reinterpret_cast<uintptr_t>(Y) % 16 == 0;
+        if (blocks || gemm) {
+            auto* base = static_cast<uint8_t*>(work);
+            auto* img = reinterpret_cast<uint2*>(base);
+            auto* fac = reinterpret_cast<float2*>(base + image_fac_offset(K));
+            auto* us = reinterpret_cast<float*>(base + image_us_offset(K));
+            const asdsl_status st = launch("batch_quantize_kernel",
+                                           group_size == 32 ? batch_quantize_kernel<32> : batch_quantize_kernel<128>,
+                                           dim3((K / 8 + 255) / 256, images * kMfmaCols), dim3(256), 0, s, X, img, fac,
+                                           gemm ? us : nullptr, K, n_cols);
+            if (st != ASDSL_OK) return st;
+            return blocks ? launch_mfma(mp, group_size, m, quant, img, fac, Y, M, K, n_cols, s)
+                          : preq2_gemm_exact(meta, quant, work, Y, M, K, group_size, n_cols, stream);
+        }
+    }
+    if (allow_mfma && n_cols >= mfma_min && mfma_ok) {
         const size_t img_bytes = static_cast<size_t>(K / 32) * kMfmaCols * 32;
         void* ws = nullptr;
         const asdsl_status st0 = work_buffer(
@@ -1084,9 +1189,9 @@ asdsl_status asdsl::preq2_fused_batch(const uint8_t* meta, const uint8_t* quant,
             const dim3 qgrid((K / 8 + 255) / 256, kMfmaCols);
             asdsl_status st = group_size == 32
                                   ? launch("batch_quantize_kernel", batch_quantize_kernel<32>, qgrid, dim3(256), 0, s,
-                                           X + static_cast<size_t>(n0) * K, img, fac, K, nc)
+                                           X + static_cast<size_t>(n0) * K, img, fac, static_cast<float*>(nullptr), K, nc)
                                   : launch("batch_quantize_kernel", batch_quantize_kernel<128>, qgrid, dim3(256), 0, s,
-                                           X + static_cast<size_t>(n0) * K, img, fac, K, nc);
+                                           X + static_cast<size_t>(n0) * K, img, fac, static_cast<float*>(nullptr), K, nc);
             if (st != ASDSL_OK) return st;
             st = launch_mfma(mp, group_size, m, quant, img, fac, Y + static_cast<size_t>(n0) * M, M, K, nc, s);
             if (st != ASDSL_OK) return st;
@@ -1343,6 +1448,11 @@ asdsl_status asdsl::preq2_batch_mfma_image(const uint8_t* meta, const uint8_t* q
 extern "C" size_t asdsl_gemv_preq2_fused_batch_work_bytes(int in_features) {
     if (in_features <= 0 || in_features % 32 != 0) return 0;
     return image_bytes(in_features);  // int8 image, group (scale, sum) pairs, slice sums
+}
+
+extern "C" size_t asdsl_gemv_preq2_fused_batch_work_bytes_n(int in_features, int n_cols) {
+    if (n_cols < 1 || n_cols > 64) return 0;
+    return (n_cols + kImageCols - 1) / kImageCols * asdsl_gemv_preq2_fused_batch_work_bytes(in_features);
 }
 
 extern "C" asdsl_status asdsl_gemv_preq2_fused_batch_ws(const uint8_t* meta, const uint8_t* quant, const float* X,

@@ -202,6 +202,12 @@ asdsl_status asdsl_gemv_preq2_fused_batch(const uint8_t* meta, const uint8_t* qu
  * in_features (any out_features and n_cols); 0 for an invalid size. */
 size_t asdsl_gemv_preq2_fused_batch_work_bytes(int in_features);
 
+/* Bytes with which asdsl_gemv_preq2_fused_batch_ws takes n_cols columns (1..64)
+ * in one pass over the weights: one activation image per 16 columns, where the
+ * size above runs them 16 at a time.  The columns' fp32 sums are then formed
+ * in asdsl_gemv_preq2_fused's order.  0 for an invalid size. */
+size_t asdsl_gemv_preq2_fused_batch_work_bytes_n(int in_features, int n_cols);
+
 /* asdsl_gemv_preq2_fused_batch with a caller-owned work buffer (256-byte
  * aligned, at least asdsl_gemv_preq2_fused_batch_work_bytes bytes; contents
  * after the call unspecified): allocates nothing.  Calls that share a work

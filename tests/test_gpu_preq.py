@@ -229,6 +229,41 @@ def test_preq2_batch_columns_do_not_depend_on_the_column_count(gpu, M, K):
             assert rel_l2(outs[n][c], outs[5][c]) < 1e-5, (n, c)
 
 
+# in_features with an MFMA tiling of up to 8 waves (operands of 4, 3 and 2
+# column blocks a launch), with one of 16 waves, and with none (ragged rows;
+# split and row-tiled exact GEMM); column counts at the edges of the blocks
+@pytest.mark.parametrize("gs,M,K,N", [
+    (32, 70, 3072, 17), (32, 257, 3072, 64), (128, 1000, 3072, 33), (32, 96, 4096, 64), (128, 64, 4096, 49),
+    (32, 129, 5120, 45), (128, 33, 5120, 64), (32, 48, 1024, 64), (128, 66, 8192, 40),
+    (32, 1003, 2688, 4), (32, 1003, 2688, 16), (128, 1001, 2944, 64), (32, 20000, 1152, 64), (128, 20002, 1152, 50),
+    (32, 50, 128, 5), (128, 50, 128, 20), (128, 38, 10240, 21)])
+def test_preq2_batch_wide(gpu, gs, M, K, N):
+    """Many columns in one call: bit for bit what 16 columns a launch give (a
+    work buffer of one image) where the MFMA kernel has a tiling, and the
+    single-column GEMV bit for bit where it has none.  Tolerance: none, the
+    same operations in the same order."""
+    import torch
+    from asdsl import _hip
+    from asdsl.kernels import _native_gemv as ng
+
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    w = torch.randn((M, K), generator=g, device="cuda", dtype=torch.float32) * 0.02
+    meta, quant = syn.preq2_from_weights_torch(w, gs)
+    X = torch.from_numpy(syn.activation(K, N, batch=N)).cuda()
+    Y, Z = (torch.full((N, M), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2))
+    ng.gemv_preq2_fused_avx2(meta, quant, X, Y, M, K, gs)
+    if K in (1024, 3072, 4096, 5120, 8192):
+        nbytes = _hip.LIB.asdsl_gemv_preq2_fused_batch_work_bytes(K)
+        work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        P = _hip.ptr
+        _hip.call("asdsl_gemv_preq2_fused_batch_ws", P(meta), P(quant), P(X), P(Z), M, K, gs, N, P(work), nbytes,
+                  _hip.stream_handle())
+    else:
+        for n in range(N):
+            ng.gemv_preq2_fused_avx2(meta, quant, X[n], Z[n], M, K, gs)
+    assert torch.equal(Y, Z)
+
+
 def test_forced_ksplit_still_covers_every_unit(gpu, monkeypatch):
     """ASDSL_HIP_KSPLIT=2 on K=8192 would leave 8 units per lane (the kernel
     takes at most 6): the plan raises the split, and the GEMV still matches
