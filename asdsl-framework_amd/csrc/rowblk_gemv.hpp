@@ -308,7 +308,13 @@ struct RowPlan {
     bool exact, multi;
 };
 
+// Layouts whose rows a wave stages through LDS (in one pass).
+template <RowLayout L>
+constexpr bool kStaged = L == RowLayout::kQ4_128 || kWideHeader<L>;
+
+template <RowLayout L>
 inline RowPlan plan_rowblk(int M, int K, int cus) {
+    using F = RowFmt<L>;
     const int U = K / 32;
     RowPlan p{4, 0, K > 4096 ? 16 : 8, 0, false, false};
     auto nu_of = [&](int llpr) { return (U + (1 << llpr) - 1) >> llpr; };
@@ -324,8 +330,23 @@ inline RowPlan plan_rowblk(int M, int K, int cus) {
         p.nu = 4;
     }
     p.exact = !p.multi && (p.nu << p.llpr) == U;
-    const int cap = cus * (32 / p.waves);  // at most 32 waves per compute unit
+    // Workgroups per compute unit.  Every workgroup stages the whole activation
+    // before its first dot, behind its own weight requests, so past the bytes
+    // that keep the memory busy a further workgroup only adds staging and
+    // contention: one where a tile holds 48 KB of weights and is staged
+    // through LDS, or where that leaves at most two tiles a workgroup; two
+    // otherwise (long rows walked in passes: up to 32 waves).  Measured
+    // against up to 32 waves per compute unit, us: Q4_K 16384x3072 9.8 -> 8.1,
+    // 24000x3072 13.5 -> 10.1, 8192x8192 17.1 -> 14.5; Q4_128 16384x3072 9.7
+    // -> 8.1, 60000x3072 22.9 -> 19.2, 200064x3072 56.2 -> 55.4, 40000x1024
+    // 7.7 -> 6.7; Q4_S256 16384x3072 9.1 -> 7.6; preq 8192x8192 10.8 -> 9.3,
+    // 40000x3072 15.5 -> 14.6.  One instead of two at smaller tiles: Q4_128
+    // 60000x1024 11.4 against 9.3; preq with more tiles: 40000x8192 38.0
+    // against 35.5.
     const int tiles = tiles_of(p.llpr);
+    const size_t tile_bytes = static_cast<size_t>(kWave >> p.llpr) * p.waves * (U / F::kUnitsPerBlock) * F::kBlockBytes;
+    const bool one = tile_bytes >= 48 * 1024 && (kStaged<L> || tiles <= 2 * cus);
+    const int cap = cus * (p.multi ? 32 / p.waves : one ? 1 : 2);
     p.grid = tiles < cap ? tiles : cap;
     return p;
 }
@@ -334,7 +355,7 @@ template <RowLayout L, int GSX, int WAVES, int NCH, bool Q8, bool EXACT, bool MU
 asdsl_status launch_rowblk_exact(const RowPlan& p, const uint8_t* blocks, const float* side, const float* x,
                                  const int8_t* xq8, const float* xsc, float* y, int M, int K, hipStream_t stream) {
     using F = RowFmt<L>;
-    constexpr bool STAGE = (L == RowLayout::kQ4_128 || kWideHeader<L>) && !MULTI;
+    constexpr bool STAGE = kStaged<L> && !MULTI;
     const size_t row_bytes = static_cast<size_t>(K / 32 / F::kUnitsPerBlock) * F::kBlockBytes;
     const size_t stage = STAGE ? WAVES * (((static_cast<size_t>(kWave >> p.llpr) * row_bytes) + 47) & ~static_cast<size_t>(15))
                                : 0;
@@ -369,7 +390,7 @@ asdsl_status launch_rowblk_waves(const RowPlan& p, const uint8_t* blocks, const 
 template <RowLayout L, int GSX, bool Q8>
 asdsl_status launch_rowblk(const uint8_t* blocks, const float* side, const float* x, const int8_t* xq8,
                            const float* xsc, float* y, int M, int K, hipStream_t stream, int cus) {
-    const RowPlan p = plan_rowblk(M, K, cus);
+    const RowPlan p = plan_rowblk<L>(M, K, cus);
     if (p.waves == 8) return launch_rowblk_waves<L, GSX, 8, 1, Q8>(p, blocks, side, x, xq8, xsc, y, M, K, stream);
     if (K <= 8192) return launch_rowblk_waves<L, GSX, 16, 1, Q8>(p, blocks, side, x, xq8, xsc, y, M, K, stream);
     if (K <= 16384) return launch_rowblk_waves<L, GSX, 16, 2, Q8>(p, blocks, side, x, xq8, xsc, y, M, K, stream);
