@@ -77,6 +77,7 @@ SIGNATURES: dict[str, list] = {
     "asdsl_gemv_sparse_unpacked": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
     "asdsl_sparse_down_proj_T": [_P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _P],
     "asdsl_sparse_down_work_bytes": [_I],
+    "asdsl_sparse_down_work_bytes_n": [_I, _I],
     "asdsl_sparse_down_proj_T_noalloc": [_P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _P],
     "asdsl_sparse_down_proj_T_ws": [_P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "asdsl_gemv_preq2_fused_batch_work_bytes": [_I],
@@ -115,7 +116,8 @@ _RESTYPE = {"asdsl_last_error": ctypes.c_char_p, "asdsl_attention_work_floats": 
             "asdsl_decode_work_bytes": ctypes.c_size_t, "asdsl_decode_verify_work_bytes": ctypes.c_size_t,
             "asdsl_decode_prefill_work_bytes": ctypes.c_size_t,
             "asdsl_decode_flags_offset": ctypes.c_size_t,
-            "asdsl_sparse_down_work_bytes": ctypes.c_size_t, "asdsl_grid_sync_probe_work_bytes": ctypes.c_size_t,
+            "asdsl_sparse_down_work_bytes": ctypes.c_size_t,
+            "asdsl_sparse_down_work_bytes_n": ctypes.c_size_t, "asdsl_grid_sync_probe_work_bytes": ctypes.c_size_t,
             "asdsl_gemv_preq2_fused_batch_work_bytes": ctypes.c_size_t,
             "asdsl_gemv_preq2_fused_batch_work_bytes_n": ctypes.c_size_t,
             "asdsl_affine_batch_work_bytes": ctypes.c_size_t}

@@ -163,6 +163,105 @@ __global__ __launch_bounds__(kWaves * kWave) void sparse_down_kernel(
     ASDSL_TIMELINE_STAMP(5, t, 4);
 }
 
+// The short list's form, one launch and no parts: workgroup = 32 outputs, its
+// kOneWaves * 64 lanes a row each (16 bytes), in passes over the list.  A
+// 128-byte line serves eight workgroups, which run on one XCD so that its L2
+// reads it once.  Each lane folds its rows in list order; the 64 lanes of a
+// wave add in a fixed halving exchange (each step hands the other half of the
+// values over, 31 exchanges for 32 sums instead of 192), the waves in order in
+// LDS.  What bounds a short list is latency (two dependent loads, a launch),
+// which the parts form pays twice; a longer one is bounded by the line lookups
+// of a compute unit (about 4 per row and workgroup), which parts spread over
+// more of them.  At 3072 outputs: 376 rows 4.2 us against 6.2 in parts, 777
+// rows 5.7 against 6.6.
+constexpr int kOneWaves = 16;
+constexpr int kOneOut = 32;
+constexpr int kOneDepth = 2;   // rows per lane in flight
+template <bool WIDE>
+__global__ __launch_bounds__(kOneWaves * kWave) void sparse_down_one_kernel(
+    const uint8_t* __restrict__ wT, const float* __restrict__ sT, const float* __restrict__ bT,
+    const float* __restrict__ x, const int32_t* __restrict__ rows, int n, float* __restrict__ y, int in_dim,
+    int out_dim, int gs) {
+    __shared__ float red[kOneWaves][kOneOut];
+    const int bid = static_cast<int>(blockIdx.x);
+    const int k = bid / kXcds;
+    const int slice = ((k / 8) * kXcds + bid % kXcds) * 8 + k % 8;  // 8 slices of a line on one XCD
+    const int o0 = slice * kOneOut;
+    if (o0 >= out_dim) return;  // the whole workgroup leaves
+    const int tid = static_cast<int>(threadIdx.x);
+    const int lane = tid & (kWave - 1);
+    const int wave = tid >> 6;
+    const int G = out_dim / gs;
+    const size_t row_bytes = static_cast<size_t>(out_dim / 2);
+    float acc[32];
+#pragma unroll
+    for (int e = 0; e < 32; ++e) acc[e] = 0.0f;
+    constexpr int stride = kOneWaves * kWave;
+    for (int a0 = tid; a0 < n; a0 += kOneDepth * stride) {
+        int r[kOneDepth];
+        float xv[kOneDepth], s[kOneDepth][4], b[kOneDepth][4];
+        uint4 w[kOneDepth];
+        bool ok[kOneDepth];
+#pragma unroll
+        for (int d = 0; d < kOneDepth; ++d) r[d] = a0 + d * stride < n ? rows[a0 + d * stride] : -1;
+#pragma unroll
+        for (int d = 0; d < kOneDepth; ++d) {
+            ok[d] = r[d] >= 0 && r[d] < in_dim;
+            const int rr = ok[d] ? r[d] : 0;  // in-bounds row for the loads below
+            xv[d] = x[rr];
+            w[d] = *reinterpret_cast<const uint4*>(wT + static_cast<size_t>(rr) * row_bytes + o0 / 2);
+#pragma unroll
+            for (int dw = 0; dw < 4; ++dw) {
+                if (WIDE && dw > 0) {
+                    s[d][dw] = s[d][0];
+                    b[d][dw] = b[d][0];
+                } else {
+                    const size_t at = static_cast<size_t>(rr) * G + (o0 + dw * 8) / gs;
+                    s[d][dw] = sT[at];
+                    b[d][dw] = bT[at];
+                }
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < kOneDepth; ++d) {
+            if (ok[d] && xv[d] != 0.0f) {
+                const uint32_t wv[4] = {w[d].x, w[d].y, w[d].z, w[d].w};
+#pragma unroll
+                for (int dw = 0; dw < 4; ++dw) {
+                    const float sx = s[d][dw] * xv[d];
+                    const float bx = b[d][dw] * xv[d];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        acc[dw * 8 + e] += fmaf(static_cast<float>((wv[dw] >> (4 * e)) & 0xFu), sx, bx);
+                }
+            }
+        }
+    }
+    // halving exchange over lane bits 5..1: lane ends with value `lane >> 1`
+    // of its half-wave pair, then bit 0 adds
+#pragma unroll
+    for (int m = 16; m >= 1; m >>= 1) {
+        const bool up = (lane & (2 * m)) != 0;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            if (e < m) {
+                const float give = up ? acc[e] : acc[e + m];
+                const float keep = up ? acc[e + m] : acc[e];
+                acc[e] = keep + __shfl_xor(give, 2 * m, kWave);
+            }
+        }
+    }
+    const float v = acc[0] + dpp<kDppQuadXor1>(acc[0]);
+    if ((lane & 1) == 0) red[wave][lane >> 1] = v;
+    __syncthreads();
+    if (tid < kOneOut) {
+        float sum = red[0][tid];
+#pragma unroll
+        for (int q = 1; q < kOneWaves; ++q) sum += red[q][tid];
+        y[o0 + tid] = sum;
+    }
+}
+
 // y[o] = part[0][o] + part[1][o] + ... + part[P-1][o], in that order.  All P
 // loads are issued before the first add, so the kernel waits on memory once.
 __global__ __launch_bounds__(64) void sparse_down_sum_parts(const float* __restrict__ part, float* __restrict__ y,
@@ -237,11 +336,27 @@ asdsl_status sparse_scratch_ptr(float** out) {
 
 struct SparsePlan {
     int nslices, nparts, per_part, grid;
+    bool one;  // sparse_down_one_kernel: no parts
 };
+
+// Short lists take the one-launch form: up to 1280 rows, or 2^21 rows x
+// outputs (device us, one launch against parts: 2048 outputs 846 rows 4.8 /
+// 6.5, 1649 rows 7.7 / 6.9; 3072 outputs 777 rows 5.7 / 6.6, 1628 rows 8.4 /
+// 7.3; 1024 outputs 2036 rows 6.6 / 7.1, 2464 rows 7.7 / 7.3).
+bool one_launch(int n_active, int out_dim) {
+    return n_active <= 1280 || static_cast<long long>(n_active) * out_dim <= (1LL << 21);
+}
 
 SparsePlan plan_sparse_down(int n_active, int out_dim, int cus) {
     SparsePlan p{};
+    p.one = one_launch(n_active, out_dim);
     p.nslices = (out_dim + kSliceOut - 1) / kSliceOut;
+    if (p.one) {
+        p.nparts = 1;
+        p.per_part = n_active;
+        p.grid = kXcds * ((p.nslices + kXcds - 1) / kXcds * 8);  // 8 workgroups per slice of kSliceOut outputs
+        return p;
+    }
     // about 3 workgroups per 4 compute units, at least 32 rows per part
     int nparts = (3 * cus / 4) / p.nslices;
     nparts = min(nparts, (n_active + kMinRowsPerPart - 1) / kMinRowsPerPart);
@@ -272,6 +387,11 @@ asdsl_status check_sparse_down(const uint8_t* w_T_packed, const float* scales_T,
 asdsl_status run_sparse_down(const SparsePlan& p, const uint8_t* w_T_packed, const float* scales_T,
                              const float* biases_T, const float* sparse_x, const int32_t* active_rows, int n_active,
                              float* y, float* part, int in_dim, int out_dim, int group_size, hipStream_t s) {
+    if (p.one)
+        return launch("sparse_down_one_kernel",
+                      group_size % 32 == 0 ? sparse_down_one_kernel<true> : sparse_down_one_kernel<false>, dim3(p.grid),
+                      dim3(kOneWaves * kWave), 0, s, w_T_packed, scales_T, biases_T, sparse_x, active_rows, n_active, y,
+                      in_dim, out_dim, group_size);
     auto kernel = group_size % 32 == 0 ? sparse_down_kernel<true> : sparse_down_kernel<false>;
     if (p.nparts == 1)
         return launch("sparse_down_kernel", kernel, dim3(p.grid), dim3(kWaves * kWave), 0, s, w_T_packed, scales_T,
@@ -289,6 +409,10 @@ asdsl_status run_sparse_down(const SparsePlan& p, const uint8_t* w_T_packed, con
 
 extern "C" size_t asdsl_sparse_down_work_bytes(int out_dim) {
     return out_dim > 0 ? static_cast<size_t>(kMaxParts) * out_dim * sizeof(float) : 0;
+}
+
+extern "C" size_t asdsl_sparse_down_work_bytes_n(int n_active, int out_dim) {
+    return n_active >= 0 && out_dim > 0 && !one_launch(n_active, out_dim) ? asdsl_sparse_down_work_bytes(out_dim) : 0;
 }
 
 extern "C" asdsl_status asdsl_sparse_down_proj_T_ws(const uint8_t* w_T_packed, const float* scales_T,

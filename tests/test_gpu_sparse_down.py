@@ -65,6 +65,29 @@ def test_shapes_and_edge_rows(gpu, IN, OUT, gs):
     assert np.all(sp.sparse_down_proj_T(wT, sT, bT, x, np.zeros(0, np.int32), IN, OUT, gs) == 0)
 
 
+# both sides of the switch between the one-launch form and the parts (1280 rows,
+# or 2^21 rows x outputs), with 8-output and 32-output scale groups, a row per
+# lane and one more, and output counts that end inside a line of 256
+@pytest.mark.parametrize("OUT,gs,n", [(1024, 32, 2048), (1024, 32, 2049), (3072, 8, 1280), (3072, 8, 1281),
+                                      (3104, 32, 1024), (2080, 16, 1025), (32, 32, 1), (288, 96, 2000)])
+def test_forms_at_their_switch(gpu, OUT, gs, n):
+    """Against the sum in float64: each output is a sum of n fp32 terms folded
+    in groups, so its error is within n * 2^-24 of the sum of the terms'
+    magnitudes; the terms are near one sign (x > 0, w around 0), and the
+    2-norm over the outputs averages to about sqrt(n) * 2^-24 < 3e-6."""
+    from asdsl.kernels import _native_sparse_gemv as sp
+
+    IN = 2100
+    wT, sT, bT = _weights(IN, OUT, gs, OUT + n)
+    rng = np.random.default_rng(n)
+    x = np.abs(rng.standard_normal(IN)).astype(np.float32) + np.float32(0.1)
+    rows = rng.permutation(IN)[:n].astype(np.int32)
+    y = sp.sparse_down_proj_T(wT, sT, bT, x, rows, IN, OUT, gs)
+    q = np.stack((wT & 15, wT >> 4), axis=-1).reshape(IN, OUT // gs, gs).astype(np.float64)
+    w = (q * sT.reshape(IN, -1, 1) + bT.reshape(IN, -1, 1)).reshape(IN, OUT)
+    assert rel_l2(y, x[rows].astype(np.float64) @ w[rows]) < 3e-6
+
+
 def test_deterministic_and_on_device(gpu):
     import torch
     from asdsl.kernels import _native_sparse_gemv as sp
