@@ -164,8 +164,8 @@ asdsl_status preq2_batch_exact_mfma_image(const uint8_t* meta, const uint8_t* qu
 // of 16 columns each (image_bytes(in_features) apart; columns past n_cols in
 // the last one may hold anything): column n of Y is bit for bit what the
 // single-column GEMV gives on column n, whatever its launch shape.
-// in_features a multiple of 128 and at most 20480; image, quant and Y 16-byte
-// aligned.
+// in_features a multiple of 128 and at most 20480; image and Y 16-byte, quant
+// and meta 4-byte aligned (as the other preq2 kernels take them).
 asdsl_status preq2_gemm_exact(const uint8_t* meta, const uint8_t* quant, const void* image, float* Y,
                               int out_features, int in_features, int group_size, int n_cols, asdsl_stream_t stream);
 

@@ -367,7 +367,7 @@ asdsl_status asdsl::preq2_gemm_exact(const uint8_t* meta, const uint8_t* quant, 
     ASDSL_CHECK_ARG((group_size == 32 || group_size == 128) && M > 0 && K > 0 && K % 128 == 0 &&
                         K / 32 <= 640 && n_cols > 0,
                     "gemm_preq2_exact: invalid dimensions");
-    ASDSL_CHECK_ARG(reinterpret_cast<uintptr_t>(image) % 16 == 0 && reinterpret_cast<uintptr_t>(quant) % 16 == 0 &&
+    ASDSL_CHECK_ARG(reinterpret_cast<uintptr_t>(image) % 16 == 0 && reinterpret_cast<uintptr_t>(quant) % 4 == 0 &&
                         reinterpret_cast<uintptr_t>(meta) % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0,
                     "gemm_preq2_exact: misaligned operand");
     ASDSL_CU_COUNT(cus);

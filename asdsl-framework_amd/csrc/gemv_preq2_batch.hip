@@ -1159,7 +1159,7 @@ asdsl_status asdsl::preq2_fused_batch(const uint8_t* meta, const uint8_t* quant,
         const bool blocks = mfma_ok && mp.waves <= 8 && n_cols > kMfmaCols && n_cols >= mfma_min;
         const bool per_column = !p.exact || K > 8192;
         const bool gemm = !mp.ok && K % 128 == 0 && n_cols >= (per_column ? 4 : 9) &&
-                          reinterpret_cast<uintptr_t>(quant) % 16 == 0 && reinterpret_cast<uintptr_t>(meta) % 4 == 0 &&
+                          reinterpret_cast<uintptr_t>(quant) % 4 == 0 && reinterpret_cast<uintptr_t>(meta) % 4 == 0 &&
                           reinterpret_cast<uintptr_t>(Y) % 16 == 0;
         if (blocks || gemm) {
             auto* base = static_cast<uint8_t*>(work);

@@ -61,12 +61,12 @@ def test_shapes(gpu, heads, kv_heads, ffn, gs_attn, gs_ffn):
 
 
 # past 2048 positions a split holds two tiles, past 4096 three
-@pytest.mark.parametrize("kv,plen", [("fp16", 2130), ("int8", 4101)])
-def test_deep_positions(gpu, kv, plen):
+@pytest.mark.parametrize("kv,kv_heads,plen", [("fp16", 4, 2130), ("int8", 4, 4101), ("int8", 2, 2070)])
+def test_deep_positions(gpu, kv, kv_heads, plen):
     from asdsl.engine import DecodeConfig
 
-    _compare(DecodeConfig(hidden=1024, n_heads=8, n_kv_heads=4, ffn=1536, vocab=2048, n_layers=2, max_seq=plen + 3,
-                          kv_format=kv), (plen,))
+    _compare(DecodeConfig(hidden=1024, n_heads=8, n_kv_heads=kv_heads, ffn=1536, vocab=2048, n_layers=2,
+                          max_seq=plen + 3, kv_format=kv), (plen,))
 
 
 def test_refused(gpu):
