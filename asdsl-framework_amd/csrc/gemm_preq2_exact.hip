@@ -34,10 +34,10 @@
 //    conflicts);
 //  - each wave's 16-row weight tile goes through its own LDS area (one 16-byte
 //    load per lane and step, read back as each MFMA's operand dwords).
-// Measured at 517 columns: gate_up 16384x3072 g128 161 us (323 T int8
+// Measured at 517 columns: gate_up 16384x3072 g128 166 us (313 T int8
 // operations a second; 15.4 vector instructions per MFMA, 70 % of the issue
-// slots taken), down 3072x8192 g128 96 us, qkv 5120x3072 g32 70 us, o_proj
-// 3072x3072 g32 44 us; the same columns as 33 launches of the 16-column exact
+// slots taken), down 3072x8192 g128 100 us, qkv 5120x3072 g32 73 us, o_proj
+// 3072x3072 g32 46 us; the same columns as 33 launches of the 16-column exact
 // kernel take 380, 280, 290 and 180 us.
 #include <cstdlib>
 
