@@ -315,8 +315,10 @@ inline int combine_threads(int max_ns) {
 // IMG_GS (32 or 128): the head's 128 outputs of column c are also quantized
 // into the o_proj batched GEMV's int8 image (image_store8, 16 chunks per
 // head, as column c0 + c of the pass), and columns at or past ncols write
-// that image's zero columns.  out may be null then.
-template <int IMG_GS>
+// that image's zero columns.
+// CHUNK: the launch's columns start at column c0 of the pass, which may hold
+// more than one image, and out may be null; otherwise c0 = 0, one image.
+template <int IMG_GS, bool CHUNK = false>
 __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const float* __restrict__ part,
                                                                       const int* __restrict__ pos_ptr, int c0,
                                                                       float* __restrict__ out, int nsplit,
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const flo
     __shared__ float gml[kCombineGroups][2];
     __shared__ float go[kCombineGroups][kHeadDim];
     __shared__ float res_s[IMG_GS != 0 ? kHeadDim : 1];
-    const int col = c0 + static_cast<int>(blockIdx.y);
+    const int col = (CHUNK ? c0 : 0) + static_cast<int>(blockIdx.y);
     const int h = static_cast<int>(blockIdx.x);
     const int tid = static_cast<int>(threadIdx.x);
     const int d = tid % kHeadDim;
@@ -338,9 +340,9 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const flo
     // the first kHeadChunks lanes quantize the head's outputs (8 each)
     auto image_chunk = [&](const float (&v)[8]) {
         if constexpr (IMG_GS != 0)
-            image_store8<IMG_GS>(v, h * kHeadChunks + tid, col % kImageCols, true, img, fac, us);
+            image_store8<IMG_GS>(v, h * kHeadChunks + tid, CHUNK ? col % kImageCols : col, true, img, fac, us);
     };
-    if constexpr (IMG_GS != 0) {
+    if constexpr (CHUNK && IMG_GS != 0) {
         const size_t at = image_at(col, static_cast<int>(gridDim.x) * kHeadDim);
         img += at / sizeof(uint2);
         fac += at / sizeof(float2);
@@ -353,9 +355,9 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const flo
     }
     const int pos = *pos_ptr + col;
     part += static_cast<size_t>(blockIdx.y) * gridDim.x * nsplit * kPartStride;
-    if (out) out += static_cast<size_t>(blockIdx.y) * gridDim.x * kHeadDim;
+    if (!CHUNK || out) out += static_cast<size_t>(blockIdx.y) * gridDim.x * kHeadDim;
     if (pos < 0 || pos >= max_seq || pos >= pos_limit) {  // no partials were written (see attn_decode_kernel)
-        if (g == 0 && out) out[static_cast<size_t>(h) * kHeadDim + d] = 0.0f;
+        if (g == 0 && (!CHUNK || out)) out[static_cast<size_t>(h) * kHeadDim + d] = 0.0f;
         if (IMG_GS != 0 && tid < kHeadChunks) image_chunk(zeros);
         return;
     }
@@ -425,7 +427,7 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(const flo
             res = sum * (1.0f / Ls);
         }
     }
-    if (g == 0 && out) out[static_cast<size_t>(h) * kHeadDim + d] = res;
+    if (g == 0 && (!CHUNK || out)) out[static_cast<size_t>(h) * kHeadDim + d] = res;
     if constexpr (IMG_GS != 0) {
         if (g == 0) res_s[d] = res;
         __syncthreads();
@@ -865,14 +867,14 @@ __global__ __launch_bounds__(256) void verify_embed_kernel(const uint16_t* __res
 // 8 wave sums in order, so both passes normalize identically.
 // IMG_GS (32 or 128): X[c] is also quantized into the next batched GEMV's
 // int8 image (image_store8, the values batch_quantize_kernel would form from
-// X; column c's image is c / kImageCols), and workgroups c >= ncols write
+// X), and workgroups c >= ncols (the grid covers kImageCols columns) write
 // that image's zero columns, so the GEMV needs no quantize launch of its own.
-// X may be null then.
+// CHUNK: more than one image of columns, and X may be null.
 // inv_out (IMG_GS = 0 only): the single-token GEMV's factored form instead,
 // X[c] = h * w and inv_out[c] = inv_rms, which the batched GEMV applies to
 // its reduced rows (preq2_batch_exact), as the norm-fed GEMV's prologue and
 // epilogue do.
-template <int IMG_GS>
+template <int IMG_GS, bool CHUNK = false>
 __global__ __launch_bounds__(kNormThreads) void verify_add_norm_kernel(float* __restrict__ H,
                                                                        const float* __restrict__ D,
                                                                        const float* __restrict__ w,
@@ -885,22 +887,25 @@ __global__ __launch_bounds__(kNormThreads) void verify_add_norm_kernel(float* __
     const int col = static_cast<int>(blockIdx.x);
     const int tid = static_cast<int>(threadIdx.x);
     const int nchunk = K >> 3;
-    if constexpr (IMG_GS != 0) {
+    if constexpr (CHUNK && IMG_GS != 0) {
         const size_t at = image_at(col, K);
         img += at / sizeof(uint2);
         fac += at / sizeof(float2);
         us += at / sizeof(float);
+    }
+    const int icol = CHUNK ? col % kImageCols : col;
+    if constexpr (IMG_GS != 0) {
         if (col >= ncols) {
             const float z[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
             for (int base = 0; base < nchunk; base += kNormThreads)  // uniform per workgroup
-                image_store8<IMG_GS>(z, base + tid, col % kImageCols, base + tid < nchunk, img, fac, us);
+                image_store8<IMG_GS>(z, base + tid, icol, base + tid < nchunk, img, fac, us);
             return;
         }
     }
     const size_t c = static_cast<size_t>(col);
     float4* h = reinterpret_cast<float4*>(H + c * K);
     const float4* d = D ? reinterpret_cast<const float4*>(D + c * K) : nullptr;
-    float4* x = X ? reinterpret_cast<float4*>(X + c * K) : nullptr;
+    float4* x = !CHUNK || X ? reinterpret_cast<float4*>(X + c * K) : nullptr;
     const float4* w4 = reinterpret_cast<const float4*>(w);
     float ss = 0.0f;
     for (int ch = tid; ch < nchunk; ch += kNormThreads) {
@@ -946,11 +951,11 @@ __global__ __launch_bounds__(kNormThreads) void verify_add_norm_kernel(float* __
         const float v[8] = {(a.x * inv_rms) * wa.x, (a.y * inv_rms) * wa.y, (a.z * inv_rms) * wa.z,
                             (a.w * inv_rms) * wa.w, (b.x * inv_rms) * wb.x, (b.y * inv_rms) * wb.y,
                             (b.z * inv_rms) * wb.z, (b.w * inv_rms) * wb.w};
-        if (x && ch < nchunk) {
+        if ((!CHUNK || x) && ch < nchunk) {
             x[2 * ch] = make_float4(v[0], v[1], v[2], v[3]);
             x[2 * ch + 1] = make_float4(v[4], v[5], v[6], v[7]);
         }
-        if constexpr (IMG_GS != 0) image_store8<IMG_GS>(v, ch, col % kImageCols, ch < nchunk, img, fac, us);
+        if constexpr (IMG_GS != 0) image_store8<IMG_GS>(v, ch, icol, ch < nchunk, img, fac, us);
     }
 }
 
@@ -1098,9 +1103,9 @@ __global__ __launch_bounds__(kAttnThreads) void verify_attn_partial_kernel(
 // (swiglu_inplace, unified_engine.cpp:803-857; the decode prologue's formula).
 // S[c] = swiglu(GU[c][0:ffn], GU[c][ffn:2ffn]), one 8-element chunk per
 // thread (grid: ceil(ffn / 2048) x columns).  IMG_GS: also the down GEMV's
-// int8 image of S (image_store8; column c's image is c / kImageCols), with
-// zero image columns for c >= ncols; S may be null then.
-template <int IMG_GS>
+// int8 image of S (image_store8), with zero image columns for c >= ncols.
+// CHUNK: more than one image of columns, and S may be null.
+template <int IMG_GS, bool CHUNK = false>
 __global__ __launch_bounds__(256) void verify_swiglu_kernel(const float* __restrict__ GU, float* __restrict__ S,
                                                             int ffn, float thr, int ncols, uint2* __restrict__ img,
                                                             float2* __restrict__ fac, float* __restrict__ us) {
@@ -1117,19 +1122,20 @@ __global__ __launch_bounds__(256) void verify_swiglu_kernel(const float* __restr
         const float* g = GU + c * 2 * ffn + 8 * cc;
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = swiglu_ref(g[e], g[ffn + e], thr);
-        if (S && ch < nchunk) {
+        if ((!CHUNK || S) && ch < nchunk) {
             float4* sp = reinterpret_cast<float4*>(S + c * ffn + 8 * ch);
             sp[0] = make_float4(v[0], v[1], v[2], v[3]);
             sp[1] = make_float4(v[4], v[5], v[6], v[7]);
         }
     }
-    if constexpr (IMG_GS != 0) {
+    if constexpr (CHUNK && IMG_GS != 0) {
         const size_t at = image_at(col, ffn);
         img += at / sizeof(uint2);
         fac += at / sizeof(float2);
         us += at / sizeof(float);
-        image_store8<IMG_GS>(v, ch, col % kImageCols, ch < nchunk, img, fac, us);
     }
+    if constexpr (IMG_GS != 0)
+        image_store8<IMG_GS>(v, ch, CHUNK ? col % kImageCols : col, ch < nchunk, img, fac, us);
 }
 
 // keys[c] = max over rows of argmax_key(logits[c][row], row): the largest
@@ -1989,7 +1995,7 @@ extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, co
                               int M, int gs) -> asdsl_status {
         const int K = m.hidden;
         const asdsl_status r = launch("verify_add_norm_kernel",
-                                      gs == 32 ? verify_add_norm_kernel<32> : verify_add_norm_kernel<128>, dim3(n),
+                                      gs == 32 ? verify_add_norm_kernel<32, true> : verify_add_norm_kernel<128, true>, dim3(n),
                                       dim3(kNormThreads), 0, s, H, D, nw, static_cast<float*>(nullptr), K, m.rms_eps,
                                       n, img, fac_of(K), us_of(K), static_cast<float*>(nullptr));
         return r != ASDSL_OK ? r : gemm(meta, quant, Y, M, K, gs);
@@ -2021,7 +2027,7 @@ extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, co
                                           m.n_heads, m.n_kv_heads, m.max_seq, w.nsplit, cus, s);
             if (st != ASDSL_OK) return st;
             if (last) break;
-            st = launch("attn_combine_kernel", m.gs_attn == 32 ? attn_combine_kernel<32> : attn_combine_kernel<128>,
+            st = launch("attn_combine_kernel", m.gs_attn == 32 ? attn_combine_kernel<32, true> : attn_combine_kernel<128, true>,
                         dim3(m.n_heads, nc), cthreads, 0, s, static_cast<const float*>(part),
                         static_cast<const int*>(pos), c0, static_cast<float*>(nullptr), w.nsplit, m.max_seq, m.max_seq,
                         0, n, kLongForm.tile, kLongForm.max_splits, img, fac_of(q_dim), us_of(q_dim));
@@ -2034,7 +2040,7 @@ extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, co
             float* down1 = base + w.down1;
             const size_t col = static_cast<size_t>(n - 1);
             const float* h = H + col * m.hidden;
-            st = launch("attn_combine_kernel", attn_combine_kernel<0>, dim3(m.n_heads), cthreads, 0, s,
+            st = launch("attn_combine_kernel", attn_combine_kernel<0, true>, dim3(m.n_heads), cthreads, 0, s,
                         static_cast<const float*>(part), static_cast<const int*>(pos), n - 1, att, w.nsplit, m.max_seq,
                         m.max_seq, 0, 1, kLongForm.tile, kLongForm.max_splits, static_cast<uint2*>(nullptr), static_cast<float2*>(nullptr),
                         static_cast<float*>(nullptr));
@@ -2062,7 +2068,7 @@ extern "C" asdsl_status asdsl_decode_prefill(const asdsl_decode_model* model, co
         if (st != ASDSL_OK) return st;
         st = norm_then_gemm(O, L.rms_ffn, L.gu_meta, L.gu_quant, GU, 2 * m.ffn, m.gs_ffn);
         if (st != ASDSL_OK) return st;
-        st = launch("verify_swiglu_kernel", m.gs_ffn == 32 ? verify_swiglu_kernel<32> : verify_swiglu_kernel<128>,
+        st = launch("verify_swiglu_kernel", m.gs_ffn == 32 ? verify_swiglu_kernel<32, true> : verify_swiglu_kernel<128, true>,
                     dim3((m.ffn / 8 + 255) / 256, n), dim3(256), 0, s, static_cast<const float*>(GU),
                     static_cast<float*>(nullptr), m.ffn, L.fatrelu_threshold, n, img, fac_of(m.ffn), us_of(m.ffn));
         if (st != ASDSL_OK) return st;
