@@ -37,8 +37,8 @@
 // Measured at 517 columns: gate_up 16384x3072 g128 166 us (313 T int8
 // operations a second; 15.4 vector instructions per MFMA, 70 % of the issue
 // slots taken), down 3072x8192 g128 100 us, qkv 5120x3072 g32 73 us, o_proj
-// 3072x3072 g32 46 us; the same columns as 33 launches of the 16-column exact
-// kernel take 380, 280, 290 and 180 us.
+// 3072x3072 g32 46 us; 33 times a launch of the 16-column exact
+// kernel would be 386, 281, 290 and 182 us.
 #include <cstdlib>
 
 #include "abi_util.hpp"
