@@ -312,6 +312,10 @@ class DecodeEngine:
         self.kv_seq_len = 0
         self._kv_snapshots: list[int] = []
         self._verify = None  # work, token, logits and next-token buffers of the verify pass
+        self._verify_n = 0  # columns of the last pass
+        # the prompt's last pass, (tokens, start), until verify_next_tokens
+        # forms its tokens; () once its K/V rows were cut or overwritten
+        self._prompt_pass: tuple | None = None
         self._prefill_work = None  # work buffer of a prefill chunk of up to _prefill_tokens tokens
         self._prefill_tokens = 0
         # ASDSL_ENGINE_PROFILE / ASDSL_ENGINE_PROFILE_TOKEN, read like the
@@ -406,6 +410,7 @@ class DecodeEngine:
                     cache[:, :ctx], L[f"{n}_scale"][:, :ctx] = kv_quantize_int8(rows)
                 else:
                     cache[:, :ctx] = rows.half()
+        self._rows_change(0)
         self.pos.fill_(ctx)
         self._host_pos = ctx
         self.kv_seq_len = ctx
@@ -427,6 +432,7 @@ class DecodeEngine:
             raise ValueError("forward_token: token_id out of vocab range")
         if not 0 <= pos < self.cfg.max_seq:
             raise ValueError("forward_token: pos out of kv-cache range")
+        self._rows_change(pos)
         self.token.fill_(token_id)
         self.pos.fill_(pos)
         limit = self._pos_limit(pos)
@@ -537,6 +543,10 @@ class DecodeEngine:
                        "asdsl_decode_prefill")
         self._host_pos = len(toks)
         self.kv_seq_len = max(self.kv_seq_len, len(toks))
+        # the last of the passes that prefill would otherwise have run
+        end = min(len(toks), self.EXACT_BATCH_LIMIT)
+        start = (end - 2) // self.MAX_VERIFY_TOKENS * self.MAX_VERIFY_TOKENS
+        self._prompt_pass = (toks[start:min(end, start + self.MAX_VERIFY_TOKENS)], start)
 
     def decode_steps(self, k: int) -> list[int]:
         """k greedy steps (step(), captured graphs) queued back to back from
@@ -572,6 +582,7 @@ class DecodeEngine:
 
         self.check_device_flags()
         self._host_pos = int(self.pos.item())
+        self._rows_change(self._host_pos)
         limit = self._pos_limit(self._host_pos)
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
@@ -610,6 +621,7 @@ class DecodeEngine:
             return
         if self._graph is None:
             self.capture()
+        self._rows_change(self._host_pos)
         self._graph.replay()
         self._host_pos += 1
 
@@ -648,6 +660,7 @@ class DecodeEngine:
         first launch's start to the last one's end; eager launches sit
         further apart than a graph's, so the span exceeds a replayed step's
         time."""
+        self._rows_change(self._host_pos)
         limit = self._pos_limit(self._host_pos) if pos_limit is None else int(pos_limit)
         stages, span = _hip.profile_stages(lambda: self._queue_step(_hip.stream_handle(), limit),
                                            max_launches=16 * self.cfg.n_layers + 16)
@@ -732,15 +745,37 @@ class DecodeEngine:
         self._host_pos = start_pos + n
         self.kv_seq_len = max(self.kv_seq_len, start_pos + n)
         self._verify_n = n
+        self._prompt_pass = None
         return v["logits"][:n]
 
     forward_verify_batch = forward_batch_all_logits
 
     def verify_next_tokens(self) -> list[int]:
-        """Greedy argmax of each column of the last multi-token pass."""
+        """Greedy argmax of each column of the last multi-token pass.  After a
+        prefill that ran in chunks, which form no logits but the last token's,
+        that is the pass over the prompt's last up to 16 tokens (from a
+        multiple of 16, below EXACT_BATCH_LIMIT) that prefill runs otherwise:
+        it is run here, at the first call, and writes its K/V rows again with
+        the bits they hold.  RuntimeError without a pass, or when those rows
+        were cut or overwritten since."""
+        if self._prompt_pass == ():
+            raise RuntimeError("verify_next_tokens: the prompt's K/V rows were cut or overwritten since its prefill")
+        if self._prompt_pass:
+            pos, host_pos, kv_len = self.pos.clone(), self._host_pos, self.kv_seq_len
+            self.forward_batch_all_logits(*self._prompt_pass)
+            self.pos.copy_(pos)
+            self._host_pos, self.kv_seq_len = host_pos, kv_len
+        if self._verify is None:
+            raise RuntimeError("verify_next_tokens: no multi-token pass yet")
         return [int(t) for t in self._verify["next"][: self._verify_n].tolist()]
 
     # ------------------------------------------------------------ KV bookkeeping
+    def _rows_change(self, from_pos: int) -> None:
+        """K/V rows from from_pos on are about to change."""
+        p = self._prompt_pass
+        if p and from_pos < p[1] + len(p[0]):
+            self._prompt_pass = ()
+
     def get_kv_seq_len(self) -> int:
         return self.kv_seq_len
 
@@ -750,6 +785,7 @@ class DecodeEngine:
         committed length (and the device position) to it."""
         c = self.cfg
         new_len = min(max(int(new_len), 0), c.max_seq)
+        self._rows_change(new_len)
         for L in self.layers:
             if self.kv_int8:
                 _hip.check(_hip.LIB.asdsl_kv_zero_from_q8(_hip.ptr(L["k_cache"]), _hip.ptr(L["v_cache"]),

@@ -78,3 +78,50 @@ def test_refused(gpu):
         eng.prefill([1, 2, 3, 4, 2048])
     with pytest.raises(ValueError, match="range"):
         eng.prefill([1] * 65)
+
+
+# 3, 4: a pass and a chunk; 17: its last pass is the first 16 tokens; 40: the
+# last 8; 2090: the pass that ends at position 2048
+@pytest.mark.parametrize("plen", [3, 4, 17, 40, 2090])
+def test_verify_next_tokens_after_a_prompt(gpu, monkeypatch, plen):
+    """The tokens of the prompt's last pass as the passes themselves give them
+    (ASDSL_HIP_VERIFY_DOT4, the pass's other form with the same bits, keeps
+    prefill on them), whatever pass came before; the K/V rows, the position
+    and the step after it as if they had not been asked for."""
+    import torch
+    from asdsl.engine import DecodeConfig, DecodeEngine
+
+    eng = DecodeEngine.synthetic(DecodeConfig(hidden=1024, n_heads=8, n_kv_heads=4, ffn=1536, vocab=2048, n_layers=2,
+                                              max_seq=2112), seed=3)
+    toks = [int(t) for t in np.random.default_rng(plen).integers(0, 2048, plen)]
+    monkeypatch.setenv("ASDSL_HIP_VERIFY_DOT4", "1")
+    eng.prefill(toks)
+    want = eng.verify_next_tokens()
+    monkeypatch.delenv("ASDSL_HIP_VERIFY_DOT4")
+    eng.reset_session()
+    eng.forward_batch_all_logits([5, 6], 0)
+    eng.prefill(toks)
+    state = _state(eng)
+    assert eng.verify_next_tokens() == want == eng.verify_next_tokens()
+    again = _state(eng)
+    assert state[1:5] == again[1:5] and torch.equal(state[0], again[0])
+    assert all(torch.equal(a, b) for a, b in zip(state[5], again[5]))
+    eng.reset_session()
+    eng.prefill(toks)
+    eng.forward_token(7, plen)  # rows after the prompt's leave it as it was
+    assert eng.verify_next_tokens() == want and eng._host_pos == plen + 1 == int(eng.pos.item())
+
+
+def test_verify_next_tokens_without_a_pass(gpu):
+    from asdsl.engine import DecodeConfig, DecodeEngine
+
+    eng = DecodeEngine.synthetic(DecodeConfig(hidden=1024, n_heads=8, n_kv_heads=4, ffn=1536, vocab=2048, n_layers=1,
+                                              max_seq=64), seed=1)
+    with pytest.raises(RuntimeError, match="no multi-token pass"):
+        eng.verify_next_tokens()
+    eng.prefill([1, 2, 3, 4, 5])
+    eng.truncate_kv(4)
+    with pytest.raises(RuntimeError, match="cut or overwritten"):
+        eng.verify_next_tokens()
+    eng.forward_batch_all_logits([3, 4, 5], 4)
+    assert len(eng.verify_next_tokens()) == 3
