@@ -531,6 +531,10 @@ class DecodeEngine:
                 raise ValueError(f"invalid decode model: {_hip.last_error()}")
             self._prefill_work = torch.empty(nbytes, dtype=torch.uint8, device=self.token.device)
             self._prefill_tokens = most
+        # A longer prompt drops the buffer while this one's launches may still
+        # be queued, on another stream than the one it was allocated on: its
+        # memory must not go to that stream's next tensor before they are done.
+        self._prefill_work.record_stream(torch.cuda.current_stream())
         ids = torch.tensor(toks, dtype=torch.int32).to(self.token.device)
         stream = _hip.stream_handle()
         for pos in range(0, len(toks), chunk):

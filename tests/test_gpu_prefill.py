@@ -125,3 +125,36 @@ def test_verify_next_tokens_without_a_pass(gpu):
         eng.verify_next_tokens()
     eng.forward_batch_all_logits([3, 4, 5], 4)
     assert len(eng.verify_next_tokens()) == 3
+
+
+def test_work_buffer_outlives_its_launches(gpu, monkeypatch):
+    """A longer prompt replaces the engine's work buffer.  While a prompt
+    queued on another stream still uses the old one, its memory is not handed
+    out again on the stream that allocated it (here at the moment the longer
+    prompt uploads its tokens, as another thread could)."""
+    import torch
+    from asdsl.engine import DecodeConfig, DecodeEngine
+
+    eng = DecodeEngine.synthetic(DecodeConfig(hidden=1024, n_heads=8, n_kv_heads=4, ffn=1536, vocab=2048, n_layers=1,
+                                              max_seq=256), seed=1)
+    eng.prefill([1] * 64)
+    torch.cuda.synchronize()
+    old = eng._prefill_work.data_ptr()
+    nbytes = eng._prefill_work.numel()
+    main, side = torch.cuda.current_stream(), torch.cuda.Stream()
+    seen = []
+    upload = torch.tensor
+
+    def tensor(*a, **k):
+        with torch.cuda.stream(main):
+            seen.append(torch.empty(nbytes, dtype=torch.uint8, device="cuda"))
+        return upload(*a, **k)
+
+    with torch.cuda.stream(side):
+        eng.prefill([2] * 64)
+        torch.cuda._sleep(200_000_000)  # the launches still queued
+        monkeypatch.setattr(torch, "tensor", tensor)
+        eng.prefill([3] * 200)
+        monkeypatch.setattr(torch, "tensor", upload)
+    assert len(seen) == 1 and seen[0].data_ptr() != old
+    torch.cuda.synchronize()
