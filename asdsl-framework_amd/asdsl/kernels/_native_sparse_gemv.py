@@ -94,7 +94,8 @@ def sparse_down_proj_T(w_T_packed, scales_T, biases_T, sparse_x, active_rows, in
     n = _numel(active_rows)
     y = new_output((out_dim,), np.float32, w_T_packed, sparse_x)
     c = DeviceCall("sparse_down_proj_T")
-    nbytes = _hip.LIB.asdsl_sparse_down_work_bytes_n(n, out_dim)
+    nbytes = (_hip.LIB.asdsl_sparse_down_work_bytes_n(n, out_dim) if group_size % 32 == 0
+              else _hip.LIB.asdsl_sparse_down_work_bytes(out_dim))
     c.run("asdsl_sparse_down_proj_T_ws", c.input(w_T_packed, np.uint8, in_dim * out_dim // 2, "w_T_packed"),
           c.input(scales_T, np.float32, in_dim * G, "scales_T"), c.input(biases_T, np.float32, in_dim * G, "biases_T"),
           c.input(sparse_x, np.float32, in_dim, "sparse_x"),

@@ -339,17 +339,38 @@ struct SparsePlan {
     bool one;  // sparse_down_one_kernel: no parts
 };
 
-// Short lists take the one-launch form: up to 1280 rows, or 2^21 rows x
-// outputs (device us, one launch against parts: 2048 outputs 846 rows 4.8 /
-// 6.5, 1649 rows 7.7 / 6.9; 3072 outputs 777 rows 5.7 / 6.6, 1628 rows 8.4 /
-// 7.3; 1024 outputs 2036 rows 6.6 / 7.1, 2464 rows 7.7 / 7.3).
-bool one_launch(int n_active, int out_dim) {
-    return n_active <= 1280 || static_cast<long long>(n_active) * out_dim <= (1LL << 21);
+// Lists that take the one-launch form.  Every workgroup of it walks the whole
+// list, so its time grows with the list's length and, past a workgroup per
+// compute unit (8192 outputs), with the outputs; the parts form takes about
+// 6 us whatever the list, 3.3 us while one part holds it (32 rows), and grows
+// later.  Us, one launch against parts, graph-replayed over one list:
+//   rows           8        32       300      700      1280      1600      2048      3000
+//   256 outputs    3.2/3.1           3.6/5.6           4.7/6.2   5.0/6.3   5.6/6.4   7.1/6.6
+//   512                              3.7/5.7           5.0/6.3   5.3/6.3   5.9/6.4   7.4/6.7
+//   1024           3.4/3.3           3.8/5.8  4.3/5.9  5.2/6.3   5.8/6.3   6.5/6.4
+//   3072           3.5/3.3           4.0/5.9  4.7/6.0  5.9/6.3
+//   8192           3.6/3.4  3.6/3.8  4.4/6.1  5.4/6.8  7.1/9.0
+//   9216                    5.2/3.8  6.4/6.2  8.2/7.3  10.9/8.8   (100 rows: 5.3/5.9)
+//   16384                   5.4/3.9  6.9/6.6  9.2/8.4  13.2/13.1  (100 rows: 5.6/6.1)
+// (with weights that no cache holds: 2048 outputs 1649 rows 7.7/6.9; 3072
+// outputs 1628 rows 8.4/7.3).  With few outputs the parts form has few slices
+// to spread its parts over, and the line lies later: 128 outputs 4096 rows
+// 6.8/6.8, 8192 rows 10.1/8.4; 64 outputs 6.5/7.0, 9.6/9.0; at 32 outputs one
+// launch stays ahead (8192 rows 9.6/13.1, 32768 rows 28.9/37.1).  Scale groups
+// of less than 32 outputs cost it four pairs a row instead of one: group 8,
+// 1024 outputs 800 rows 6.4/7.0, 1280 rows 8.5/7.3; 5120 outputs 700 rows
+// 7.0/7.7, 800 rows 7.8/7.9; 8192 outputs 500 rows 7.4/7.8, 700 rows 8.9/8.3.
+bool one_launch(int n_active, int out_dim, int gs) {
+    if (out_dim > 8192) return n_active > kMinRowsPerPart && n_active <= 200;
+    if (n_active <= 16) return false;
+    if (gs % 32 != 0) return n_active <= (out_dim <= 5120 ? 800 : 600);
+    const int most = out_dim <= 32 ? 61440 : out_dim <= 128 ? 4096 : 2048;
+    return n_active <= 1280 || (n_active <= most && static_cast<long long>(n_active) * out_dim <= 1920LL * 1024);
 }
 
-SparsePlan plan_sparse_down(int n_active, int out_dim, int cus) {
+SparsePlan plan_sparse_down(int n_active, int out_dim, int gs, int cus) {
     SparsePlan p{};
-    p.one = one_launch(n_active, out_dim);
+    p.one = one_launch(n_active, out_dim, gs);
     p.nslices = (out_dim + kSliceOut - 1) / kSliceOut;
     if (p.one) {
         p.nparts = 1;
@@ -412,7 +433,8 @@ extern "C" size_t asdsl_sparse_down_work_bytes(int out_dim) {
 }
 
 extern "C" size_t asdsl_sparse_down_work_bytes_n(int n_active, int out_dim) {
-    return n_active >= 0 && out_dim > 0 && !one_launch(n_active, out_dim) ? asdsl_sparse_down_work_bytes(out_dim) : 0;
+    if (n_active <= kMinRowsPerPart || out_dim <= 0 || one_launch(n_active, out_dim, 32)) return 0;
+    return asdsl_sparse_down_work_bytes(out_dim);
 }
 
 extern "C" asdsl_status asdsl_sparse_down_proj_T_ws(const uint8_t* w_T_packed, const float* scales_T,
@@ -427,7 +449,7 @@ extern "C" asdsl_status asdsl_sparse_down_proj_T_ws(const uint8_t* w_T_packed, c
                     "sparse_down_proj_T: work buffer of %zu bytes, asdsl_sparse_down_work_bytes gives %zu", work_bytes,
                     asdsl_sparse_down_work_bytes(out_dim));
     ASDSL_CU_COUNT(cus);
-    const SparsePlan p = plan_sparse_down(n_active, out_dim, cus);
+    const SparsePlan p = plan_sparse_down(n_active, out_dim, group_size, cus);
     hipStream_t s = as_hip(stream);
     void* part = nullptr;
     if (p.nparts > 1) {
@@ -458,7 +480,7 @@ extern "C" asdsl_status asdsl_sparse_down_proj_T_noalloc(const uint8_t* w_T_pack
     ASDSL_CHECK_ARG(out_dim <= kNoAllocMaxOut, "sparse_down_proj_T_noalloc: out_dim %d exceeds the %d outputs of its "
                     "device scratch array", out_dim, kNoAllocMaxOut);
     ASDSL_CU_COUNT(cus);
-    const SparsePlan p = plan_sparse_down(n_active, out_dim, cus);
+    const SparsePlan p = plan_sparse_down(n_active, out_dim, group_size, cus);
     float* part = nullptr;
     if (p.nparts > 1) {
         const asdsl_status st = sparse_scratch_ptr(&part);

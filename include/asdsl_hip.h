@@ -396,8 +396,10 @@ asdsl_status asdsl_sparse_down_proj_T(const uint8_t* w_T_packed, const float* sc
  * (any list length); 0 for out_dim <= 0. */
 size_t asdsl_sparse_down_work_bytes(int out_dim);
 
-/* The same for a call with n_active listed rows: 0 where it needs none (a
- * short list; work may then be null, and the library's buffer is not used). */
+/* The same for a call with n_active listed rows and a group_size that is a
+ * multiple of 32: 0 where it needs none (a short list, or an invalid size):
+ * work is then null, and the library's buffer is not used.  A work pointer
+ * that is not null has the size above, whatever the list. */
 size_t asdsl_sparse_down_work_bytes_n(int n_active, int out_dim);
 
 /* asdsl_sparse_down_proj_T with a caller-owned work buffer (256-byte aligned,

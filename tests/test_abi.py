@@ -103,6 +103,12 @@ def test_work_buffer_queries_and_checks_without_gpu():
     one = ctypes.c_void_p(256)
     assert lib.asdsl_sparse_down_work_bytes(3072) == 32 * 3072 * 4
     assert lib.asdsl_sparse_down_work_bytes(0) == 0
+    # a list needs no work buffer where one launch takes it (the faster form there) or one part of 32 rows holds it
+    for n, out, none in ((0, 3072, True), (32, 16384, True), (33, 16384, True), (200, 16384, True), (201, 16384, False),
+                         (1280, 8192, True), (1281, 3072, False), (1920, 1024, True), (1921, 1024, False),
+                         (2048, 512, True), (2049, 512, False), (8192, 256, False), (4096, 128, True),
+                         (4097, 64, False), (32768, 32, True), (-1, 1024, True), (5000, 0, True)):
+        assert lib.asdsl_sparse_down_work_bytes_n(n, out) == (0 if none else 32 * out * 4), (n, out)
     # per 32-element slice and column: 32 int8 codes, a (scale, sum) pair, a slice sum
     assert lib.asdsl_gemv_preq2_fused_batch_work_bytes(3072) == 96 * 16 * 44
     assert lib.asdsl_gemv_preq2_fused_batch_work_bytes(100) == 0

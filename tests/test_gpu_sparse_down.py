@@ -88,6 +88,30 @@ def test_forms_at_their_switch(gpu, OUT, gs, n):
     assert rel_l2(y, x[rows].astype(np.float64) @ w[rows]) < 3e-6
 
 
+# the row limits of the one-launch form and one row past each: 17 rows; 2048,
+# 4096 up to 128 outputs, 1920 x 1024 rows x outputs; groups of less than 32
+# outputs 800 rows, 600 past 5120 outputs; 33 to 200 rows past 8192 outputs; 32
+# outputs keep it for long lists
+@pytest.mark.parametrize("OUT,gs,n", [(1024, 32, 16), (1024, 32, 17), (1024, 32, 1920), (1024, 32, 1921),
+                                      (256, 32, 2048), (256, 32, 2049), (128, 32, 4096), (128, 32, 4097),
+                                      (32, 32, 9001), (96, 8, 800), (96, 8, 801), (5152, 16, 600), (5152, 16, 601),
+                                      (8224, 32, 32), (8224, 32, 33), (8224, 32, 200), (8224, 32, 201)])
+def test_forms_at_the_row_limits(gpu, OUT, gs, n):
+    """Against the sum in float64: 2^-24 * sqrt(n) of the terms' magnitudes
+    (see test_forms_at_their_switch), 5.7e-6 at n = 9001."""
+    from asdsl.kernels import _native_sparse_gemv as sp
+
+    IN = n + 7
+    wT, sT, bT = _weights(IN, OUT, gs, OUT + n)
+    rng = np.random.default_rng(n)
+    x = np.abs(rng.standard_normal(IN)).astype(np.float32) + np.float32(0.1)
+    rows = rng.permutation(IN)[:n].astype(np.int32)
+    y = sp.sparse_down_proj_T(wT, sT, bT, x, rows, IN, OUT, gs)
+    q = np.stack((wT & 15, wT >> 4), axis=-1).reshape(IN, OUT // gs, gs).astype(np.float64)
+    w = (q * sT.reshape(IN, -1, 1) + bT.reshape(IN, -1, 1)).reshape(IN, OUT)
+    assert rel_l2(y, x[rows].astype(np.float64) @ w[rows]) < 5.7e-6
+
+
 def test_deterministic_and_on_device(gpu):
     import torch
     from asdsl.kernels import _native_sparse_gemv as sp
