@@ -312,7 +312,7 @@ struct RowPlan {
 template <RowLayout L>
 constexpr bool kStaged = L == RowLayout::kQ4_128 || kWideHeader<L>;
 
-template <RowLayout L>
+template <RowLayout L, bool Q8>
 inline RowPlan plan_rowblk(int M, int K, int cus) {
     using F = RowFmt<L>;
     const int U = K / 32;
@@ -334,19 +334,41 @@ inline RowPlan plan_rowblk(int M, int K, int cus) {
     // before its first dot, behind its own weight requests, so past the bytes
     // that keep the memory busy a further workgroup only adds staging and
     // contention: one where a tile holds 48 KB of weights and is staged
-    // through LDS, or where that leaves at most two tiles a workgroup; two
-    // otherwise (long rows walked in passes: up to 32 waves).  Measured
-    // against up to 32 waves per compute unit, us: Q4_K 16384x3072 9.8 -> 8.1,
-    // 24000x3072 13.5 -> 10.1, 8192x8192 17.1 -> 14.5; Q4_128 16384x3072 9.7
-    // -> 8.1, 60000x3072 22.9 -> 19.2, 200064x3072 56.2 -> 55.4, 40000x1024
-    // 7.7 -> 6.7; Q4_S256 16384x3072 9.1 -> 7.6; preq 8192x8192 10.8 -> 9.3,
-    // 40000x3072 15.5 -> 14.6.  One instead of two at smaller tiles: Q4_128
-    // 60000x1024 11.4 against 9.3; preq with more tiles: 40000x8192 38.0
-    // against 35.5.
+    // through LDS, or where that leaves at most two tiles a workgroup (not
+    // with 8 waves and the activation quantized beforehand, which is little to
+    // stage: preq 16384x3072 8.2 against 7.9); two otherwise (long rows walked
+    // in passes: up to 32 waves).  Measured against up to 32 waves per compute
+    // unit, us: Q4_K 16384x3072 9.8 -> 8.1, 24000x3072 13.5 -> 10.1, 8192x8192
+    // 17.1 -> 14.5; Q4_128 16384x3072 9.5 -> 7.9, 60000x3072 22.6 -> 19.7,
+    // 200064x3072 56.1 -> 52.4, 40000x1024 7.5 -> 6.6; Q4_S256 16384x3072 9.1
+    // -> 7.6; preq 8192x8192 10.8 -> 9.3, 40000x3072 15.5 -> 14.6.  One instead
+    // of two at smaller tiles: Q4_128 60000x1024 11.4 against 9.3; preq with
+    // more tiles: 40000x8192 38.0 against 35.5.
     const int tiles = tiles_of(p.llpr);
     const size_t tile_bytes = static_cast<size_t>(kWave >> p.llpr) * p.waves * (U / F::kUnitsPerBlock) * F::kBlockBytes;
-    const bool one = tile_bytes >= 48 * 1024 && (kStaged<L> || tiles <= 2 * cus);
-    const int cap = cus * (p.multi ? 32 / p.waves : one ? 1 : 2);
+    const bool one = tile_bytes >= 48 * 1024 && (kStaged<L> || (tiles <= 2 * cus && !(Q8 && p.waves == 8)));
+    // Up to 32 waves again once many tiles have amortized the staging, where
+    // a wave's own chain of loads is what its tile then waits for (us, 32
+    // waves against two workgroups):
+    //  - rows of at most one unit per lane (512 elements), tiles of 5 to 10 KB:
+    //    Q4_128 200064x512 14.9 / 17.0, 60000x512 6.5 / 7.1, 30000x512 4.7 /
+    //    4.8; with staging and the activation quantized beforehand from 3 tiles
+    //    a compute unit, Q4_S256 30000x256 3.9 / 4.1;
+    //  - layouts read straight from memory, with little to stage (quantized
+    //    beforehand, or packed): rows of two units per lane (1024 elements), preq
+    //    80000x768 8.3 / 8.7, packed g128 80000x768 7.3 / 7.8 (preq quantizing
+    //    itself 200064x1024 23.8 / 23.0); longer ones in tiles of 20 KB and more,
+    //    preq 130000x1280 18.6 / 19.4, packed g128 80000x1280 10.1 / 10.4;
+    //  - preq quantizing itself and Q4_S256 at tiles of 24 KB and more: preq
+    //    200064x1280 26.5 / 27.7, 80000x4096 35.3 / 36.7, 30000x4096 15.0 / 14.7;
+    //    Q4_S256 130000x4096 47.5 / 48.9, 30000x4096 14.3 / 14.0; Q4_128
+    //    130000x4096 49.3 / 48.1.
+    constexpr bool kLight = !kStaged<L> && (Q8 || L == RowLayout::kPacked);
+    bool many = false;
+    if (p.nu == 1) many = tiles > (Q8 && kStaged<L> ? 3 : 6) * cus;
+    else if (kLight && p.nu == 2) many = tiles > 6 * cus;
+    else if (!kStaged<L> || L == RowLayout::kQ4S256) many = tile_bytes >= (kLight ? 20 : 24) * 1024 && tiles > (kLight ? 8 : 10) * cus;
+    const int cap = cus * (p.multi ? 32 / p.waves : one ? 1 : many ? 32 / p.waves : 2);
     p.grid = tiles < cap ? tiles : cap;
     return p;
 }
@@ -390,7 +412,7 @@ asdsl_status launch_rowblk_waves(const RowPlan& p, const uint8_t* blocks, const 
 template <RowLayout L, int GSX, bool Q8>
 asdsl_status launch_rowblk(const uint8_t* blocks, const float* side, const float* x, const int8_t* xq8,
                            const float* xsc, float* y, int M, int K, hipStream_t stream, int cus) {
-    const RowPlan p = plan_rowblk<L>(M, K, cus);
+    const RowPlan p = plan_rowblk<L, Q8>(M, K, cus);
     if (p.waves == 8) return launch_rowblk_waves<L, GSX, 8, 1, Q8>(p, blocks, side, x, xq8, xsc, y, M, K, stream);
     if (K <= 8192) return launch_rowblk_waves<L, GSX, 16, 1, Q8>(p, blocks, side, x, xq8, xsc, y, M, K, stream);
     if (K <= 16384) return launch_rowblk_waves<L, GSX, 16, 2, Q8>(p, blocks, side, x, xq8, xsc, y, M, K, stream);
