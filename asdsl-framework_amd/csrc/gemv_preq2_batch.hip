@@ -1150,15 +1150,19 @@ asdsl_status asdsl::preq2_fused_batch(const uint8_t* meta, const uint8_t* quant,
     //    14.3).  16-wave tilings (in_features 8192) have no registers for a
     //    second block and stay at 16 columns a launch;
     //  - no MFMA tiling for in_features: the exact GEMM, the single-column
-    //    GEMV's bits, where that would otherwise run once per column (3.3 us
-    //    each: from 4 columns; 1000x2688 g32 at 4 / 45 columns: 13.4 / 148 ->
-    //    7.8 / 8.3 us) or as dot4 launches of 8 columns (beyond 8; 16384x1536
-    //    g32 at 8 / 16 / 45: dot4 11.3 / 22.1 / 62, the GEMM 10.9 / 11.0 / 19.6).
+    //    GEMV's bits, where that would otherwise run once per column (3.5 us
+    //    each: from 4 columns; 1000x2688 g32 at 4 / 45 columns: 14.6 / 158 ->
+    //    7.8 / 8.1 us.  Its steps are a serial chain along in_features, so with
+    //    rows longer than 10240 and too few of them to fill the chip from 5:
+    //    1000x20480 g32 at 4 / 5: 24.7 / 30.6, the GEMM 28.7 / 28.6; 4096x20480
+    //    at 4: 44.4, the GEMM 33.3) or as dot4 launches of 8 columns (beyond 8;
+    //    16384x1536 g32 at 8 / 9 / 16 / 45: dot4 12.1 / 16.5 / 23.8 / 67, the GEMM
+    //    from 9: 9.4 / 9.6 / 19.7).
     const int images = (n_cols + kMfmaCols - 1) / kMfmaCols;
     if (allow_mfma && work && work_bytes >= images * image_bytes(K) && reinterpret_cast<uintptr_t>(work) % 256 == 0) {
         const bool blocks = mfma_ok && mp.waves <= 8 && n_cols > kMfmaCols && n_cols >= mfma_min;
         const bool per_column = !p.exact || K > 8192;
-        const bool gemm = !mp.ok && K % 128 == 0 && n_cols >= (per_column ? 4 : 9) &&
+        const bool gemm = !mp.ok && K % 128 == 0 && n_cols >= (!per_column ? 9 : K > 10240 && M <= 1024 ? 5 : 4) &&
                           reinterpret_cast<uintptr_t>(quant) % 4 == 0 && reinterpret_cast<uintptr_t>(meta) % 4 == 0 &&
                           reinterpret_cast<uintptr_t>(Y) % 16 == 0;
         if (blocks || gemm) {

@@ -264,6 +264,47 @@ def test_preq2_batch_wide(gpu, gs, M, K, N):
     assert torch.equal(Y, Z)
 
 
+# rows longer than 10240: up to 1024 of them run 4 columns one by one and 5
+# together, more of them 4 together
+@pytest.mark.parametrize("gs,M,K,N", [(32, 1000, 20480, 4), (32, 1000, 20480, 5), (128, 1025, 10368, 4)])
+def test_preq2_batch_long_rows(gpu, gs, M, K, N):
+    """The single-column GEMV bit for bit.  Tolerance: none."""
+    import torch
+    from asdsl.kernels import _native_gemv as ng
+
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    meta, quant = syn.preq2_from_weights_torch(torch.randn((M, K), generator=g, device="cuda") * 0.02, gs)
+    X = torch.from_numpy(syn.activation(K, N, batch=N)).cuda()
+    Y, Z = (torch.full((N, M), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2))
+    ng.gemv_preq2_fused_avx2(meta, quant, X, Y, M, K, gs)
+    for n in range(N):
+        ng.gemv_preq2_fused_avx2(meta, quant, X[n], Z[n], M, K, gs)
+    assert torch.equal(Y, Z)
+
+
+# column blocks in one MFMA launch, which has no need of an aligned Y, and the
+# exact GEMM, which leaves such a call to the single-column GEMV; odd and even
+# numbers of rows
+@pytest.mark.parametrize("M,K,N", [(257, 3072, 33), (1003, 2688, 20), (256, 2688, 9)])
+def test_preq2_batch_wide_with_a_misaligned_result(gpu, M, K, N):
+    """A result 4 bytes past a 16-byte boundary: the bits of an aligned one,
+    and nothing written around it.  Tolerance: none."""
+    import torch
+    from asdsl.kernels import _native_gemv as ng
+
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    meta, quant = syn.preq2_from_weights_torch(torch.randn((M, K), generator=g, device="cuda") * 0.02, 32)
+    X = torch.from_numpy(syn.activation(K, N, batch=N)).cuda()
+    Y = torch.empty((N, M), device="cuda")
+    ng.gemv_preq2_fused_avx2(meta, quant, X, Y, M, K, 32)
+    buf = torch.full((N * M + 8,), float("nan"), device="cuda")
+    out = buf[1:1 + N * M].view(N, M)
+    assert out.data_ptr() % 16 == 4
+    ng.gemv_preq2_fused_avx2(meta, quant, X, out, M, K, 32)
+    assert torch.equal(out, Y)
+    assert torch.isnan(buf[0]) and torch.isnan(buf[1 + N * M:]).all()
+
+
 def test_forced_ksplit_still_covers_every_unit(gpu, monkeypatch):
     """ASDSL_HIP_KSPLIT=2 on K=8192 would leave 8 units per lane (the kernel
     takes at most 6): the plan raises the split, and the GEMV still matches
