@@ -202,10 +202,19 @@ asdsl_status asdsl_gemv_preq2_fused_batch(const uint8_t* meta, const uint8_t* qu
  * in_features (any out_features and n_cols); 0 for an invalid size. */
 size_t asdsl_gemv_preq2_fused_batch_work_bytes(int in_features);
 
-/* Bytes with which asdsl_gemv_preq2_fused_batch_ws takes n_cols columns (1..64)
- * in one pass over the weights: one activation image per 16 columns, where the
- * size above runs them 16 at a time.  The columns' fp32 sums are then formed
- * in asdsl_gemv_preq2_fused's order.  0 for an invalid size. */
+/* Bytes with which asdsl_gemv_preq2_fused_batch_ws may take n_cols columns
+ * (1..64) together: one activation image per 16 columns, where the size above
+ * runs them 16 at a time.  With this room, and every operand aligned:
+ *  - more than 16 columns, in_features 2048, 3072, 4096 or 5120, and 1024 at
+ *    group_size 32: the weights are read once for up to 64 columns (48 or 32
+ *    where more leave too few registers), each column with the bits of 16
+ *    columns a call;
+ *  - in_features 8192, and 6144 at group_size 32: 16 columns a pass, as without
+ *    it;
+ *  - other multiples of 128, from 4 columns (5 or 9 where the other forms are
+ *    faster): one pass, each column with asdsl_gemv_preq2_fused's bits; with
+ *    fewer columns as without it.
+ * 0 for an invalid size. */
 size_t asdsl_gemv_preq2_fused_batch_work_bytes_n(int in_features, int n_cols);
 
 /* asdsl_gemv_preq2_fused_batch with a caller-owned work buffer (256-byte
@@ -611,7 +620,11 @@ size_t asdsl_decode_prefill_work_bytes(const asdsl_decode_model* model, int max_
  * Writes the chunk's K/V rows; with logits (device [vocab], may be null) also
  * the last token's logits and *token = their greedy argmax; *pos = start_pos +
  * n (device ints; *pos is used as scratch meanwhile).  What it writes is what
- * asdsl_decode_token on each token in turn leaves, bit for bit.  1 <= n <=
+ * asdsl_decode_token_upto on each token in turn leaves, bit for bit, with a
+ * pos_limit of at most 2048 for positions below 2048 and a larger one from
+ * there on.  (asdsl_decode_token on a cache of more than 2048 positions takes
+ * the larger limit everywhere: below 2048 its attention sums in another order,
+ * and the two agree to fp32 rounding.)  1 <= n <=
  * 1024, start_pos + n <= max_seq; work: asdsl_decode_prefill_work_bytes(model,
  * >= n) bytes, 256-byte aligned.  ASDSL_ERR_UNSUPPORTED (nothing queued) under
  * ASDSL_HIP_NORM_FACTORED.  The reference feeds a prompt one forward_token
