@@ -637,12 +637,12 @@ Plan plan_preq2(int M, int K, int cus, int gs) {
     p.exact = p.nu * (kWave << p.lks) == upb;
     // At most 32 waves per compute unit; half of that, so that half as many
     // workgroups stage the activation, up to 6 tiles per compute unit (us: 8
-    // waves 24000x3072 g32 10.3 -> 9.1, 40000x3072 14.8 -> 13.6, 12000x4096
-    // 7.8 -> 7.0; 16 waves 8192x8192 10.7 -> 9.4, 24000x8192 22.2 -> 21.0).
+    // waves 24000x3072 g32 10.2 -> 9.3, 40000x3072 14.7 -> 13.7, 12000x4096
+    // 7.8 -> 6.9; 16 waves 8192x8192 10.7 -> 9.4, 24000x8192 21.9 -> 20.7).
     // With more tiles per workgroup the staging is amortized anyway, and more
     // waves hide the end of a tile better (60000x1024 g128 7.4, halved 8.0).
     const int tiles = tiles_of(p.lks);
-    const int cap = cus * (32 / p.waves) / (tiles <= 6 * cus && p.waves != 12 ? 2 : 1);
+    const int cap = cus * (32 / p.waves) / (tiles <= 6 * cus ? 2 : 1);
     p.grid = tiles < cap ? tiles : cap;
     // The activation waits in the memory queues behind the weight requests
     // issued before it, so its arrival grows with the bytes a launch
