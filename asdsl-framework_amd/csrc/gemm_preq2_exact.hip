@@ -21,7 +21,9 @@
 // What bounds it: the fp32 steps.  Per MFMA each lane forms 4 values with 4
 // conversions, 4 products s*xs (one in four of them for GS 128) and 8 fused
 // multiply-adds on the vector unit, 13-16 instructions of 4 cycles against 16
-// matrix cycles.  So the kernel keeps everything else off the vector unit:
+// matrix cycles; decoding (s, -z*s), unpacking weights and addresses add
+// 5 to 8.  So the kernel keeps what it can off the
+// vector unit:
 //  - the MFMA's rows are the weight rows and its columns the activation
 //    columns: a lane holds one column's (xs, xu) and four rows' (s, z), and
 //    one unpacked weight operand serves CB column blocks;
@@ -29,15 +31,16 @@
 //    activation operands and scales of a step are staged once in LDS for all
 //    of them (two buffers, the next step's loads in flight while the current
 //    one computes; one barrier per step);
-//    Both are laid out in LDS so that no two lanes of a read share a bank
-//    (as first written, 41 % of the cycles of a gate_up launch were bank
-//    conflicts);
+//    Both are laid out in LDS so that no two lanes of an operand read share
+//    a bank (as first written, 41 % of the cycles of a gate_up launch were
+//    bank conflicts; 6 % are left, the operands' stores among them, whose two
+//    halves of a unit fall on the same banks);
 //  - each wave's 16-row weight tile goes through its own LDS area (one 16-byte
 //    load per lane and step, read back as each MFMA's operand dwords).
 // Measured at 517 columns: gate_up 16384x3072 g128 166 us (313 T int8
-// operations a second; 15.4 vector instructions per MFMA, 70 % of the issue
-// slots taken), down 3072x8192 g128 100 us, qkv 5120x3072 g32 73 us, o_proj
-// 3072x3072 g32 46 us; 33 times a launch of the 16-column exact
+// operations a second; 18.5 vector instructions beside each MFMA, 70 % of the
+// issue slots taken), down 3072x8192 g128 100 us, qkv 5120x3072 g32 73 us (22.7 beside
+// each MFMA), o_proj 3072x3072 g32 46 us; 33 times a launch of the 16-column exact
 // kernel would be 386, 281, 290 and 182 us.
 #include <cstdlib>
 

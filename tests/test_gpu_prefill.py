@@ -69,6 +69,64 @@ def test_deep_positions(gpu, kv, kv_heads, plen):
                           max_seq=plen + 3, kv_format=kv), (plen,))
 
 
+# three query heads per KV head past 2048 positions, fp16 rows
+def test_deep_positions_three_heads(gpu):
+    from asdsl.engine import DecodeConfig
+
+    _compare(DecodeConfig(hidden=768, n_heads=6, n_kv_heads=2, ffn=1536, vocab=2048, n_layers=2, max_seq=2100), (2085,))
+
+
+# chunks of up to 16 tokens at positions past 0: the projections' 16-column form
+# (every in_features of the first model has it) and the GEMM's split form
+@pytest.mark.parametrize("hidden,heads,kv_heads,ffn", [(3072, 24, 8, 8192), (1024, 8, 4, 3712)])
+def test_short_chunks(gpu, monkeypatch, hidden, heads, kv_heads, ffn):
+    from asdsl.engine import DecodeConfig, DecodeEngine
+
+    monkeypatch.setattr(DecodeEngine, "MAX_PREFILL_TOKENS", 16)
+    _compare(DecodeConfig(hidden=hidden, n_heads=heads, n_kv_heads=kv_heads, ffn=ffn, vocab=1003, n_layers=2,
+                          max_seq=64), (17, 40))
+
+
+@pytest.mark.parametrize("switch", ["ASDSL_HIP_VERIFY_DOT4", "ASDSL_HIP_NORM_FACTORED"])
+def test_prompts_under_the_switches(gpu, monkeypatch, switch):
+    """Prompts that run as verify passes of up to 16 tokens (16 + a single
+    step, 16 + 16 + 8) and single steps past position 2048, against
+    forward_token under the same switch."""
+    from asdsl.engine import DecodeConfig, DecodeEngine
+
+    monkeypatch.setenv(switch, "1")
+    monkeypatch.setattr(DecodeEngine, "_prefill_chunks", None)  # not called
+    _compare(DecodeConfig(hidden=1024, n_heads=8, n_kv_heads=4, ffn=1536, vocab=2048, n_layers=2, max_seq=2112),
+             (17, 40, 2051))
+
+
+def test_refused_by_the_library(gpu, monkeypatch):
+    """asdsl_decode_prefill's argument checks; nothing is queued."""
+    import ctypes
+
+    import torch
+    from asdsl import _hip
+    from asdsl.engine import DecodeConfig, DecodeEngine
+
+    eng = DecodeEngine.synthetic(DecodeConfig(hidden=1024, n_heads=8, n_kv_heads=4, ffn=1536, vocab=2048, n_layers=1,
+                                              max_seq=64), seed=1)
+    eng.prefill([1, 2, 3, 4])
+    lib, model, P = _hip.LIB, ctypes.byref(eng._model), _hip.ptr
+    ids = torch.ones(64, dtype=torch.int32, device="cuda")
+
+    def call(n=4, start=0, work=0, tokens=None, logits=None):
+        return lib.asdsl_decode_prefill(model, P(ids) if tokens is None else tokens, n, start, P(eng.token),
+                                        P(eng.pos), logits, P(eng._prefill_work) + work, _hip.stream_handle())
+
+    bad = _hip.ASDSL_ERR_INVALID_ARGUMENT
+    assert lib.asdsl_decode_prefill_work_bytes(model, 0) == lib.asdsl_decode_prefill_work_bytes(model, 1025) == 0
+    assert lib.asdsl_decode_prefill_work_bytes(None, 4) == 0
+    assert call(n=0) == call(n=1025) == call(start=-1) == call(start=61) == call(work=64) == call(tokens=0) == bad
+    monkeypatch.setenv("ASDSL_HIP_NORM_FACTORED", "1")
+    assert call() not in (bad, 0) and "factored" in _hip.last_error()
+    assert int(eng.pos.item()) == 4
+
+
 def test_refused(gpu):
     from asdsl.engine import DecodeConfig, DecodeEngine
 

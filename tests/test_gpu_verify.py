@@ -444,11 +444,11 @@ def test_reference_calls_replay_graphs_with_the_eager_bits(gpu, monkeypatch):
 
 @pytest.mark.parametrize("kv", ["fp16", "int8"])
 def test_prefill_is_forward_token_on_each_token(gpu, kv):
-    """DecodeEngine.prefill runs a prompt as verify passes of up to 16
-    tokens: K/V rows, logits of the last token, device token, position and
-    KV length as forward_token on each prompt token in turn leaves them, bit
-    for bit, for prompts of 1 to 40 tokens (single step, a 2-token pass, 16,
-    16 + 1 single step, 16 + 16 + 8)."""
+    """DecodeEngine.prefill: K/V rows, logits of the last token, device
+    token, position and KV length as forward_token on each prompt token in
+    turn leaves them, bit for bit, for prompts of 1 to 40 tokens (a single
+    step, a 2-token pass, chunks from 4 tokens; test_gpu_prefill.py runs the
+    passes on longer prompts)."""
     import torch
     from asdsl.engine import DecodeConfig, DecodeEngine
 
