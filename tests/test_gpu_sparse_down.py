@@ -65,9 +65,10 @@ def test_shapes_and_edge_rows(gpu, IN, OUT, gs):
     assert np.all(sp.sparse_down_proj_T(wT, sT, bT, x, np.zeros(0, np.int32), IN, OUT, gs) == 0)
 
 
-# the one-launch form up to 1280 rows and the parts beyond, with 8-output,
-# 16-output and 32-output scale groups, a row per lane and one more, and output
-# counts that end inside a line of 256 (its limits: test_forms_at_the_row_limits)
+# the parts form at 1025 to 2049 rows with 8-output, 16-output and 32-output scale
+# groups, the one-launch form with a row per lane of a workgroup and with groups
+# of 96, and output counts that end inside a line of 256 (the line between the
+# forms: test_forms_at_the_row_limits)
 @pytest.mark.parametrize("OUT,gs,n", [(1024, 32, 2048), (1024, 32, 2049), (3072, 8, 1280), (3072, 8, 1281),
                                       (3104, 32, 1024), (2080, 16, 1025), (32, 32, 1), (288, 96, 2000)])
 def test_forms_at_their_switch(gpu, OUT, gs, n):
